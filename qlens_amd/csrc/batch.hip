@@ -21,8 +21,12 @@
 //   model, chi^2, Es         lens.cpp:12950-13015, pixelgrid.cpp:15821-15863, 18268-18307
 #include "qlx_internal.h"
 
+#include <type_traits>
+#include <utility>
+
 namespace qlx {
 
+typedef double double2_t __attribute__((ext_vector_type(2)));
 typedef double double4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -1603,8 +1607,8 @@ void launch_prep_fr_b(hipStream_t s, const BatchDev& bd, int max_ld, int f32)
 
 // ------------------------------------------------------------------------------------------------
 // Batched blocked Cholesky (lower, 64x64 tiles) of many matrices, FP64 or FP32 per matrix, dense
-// or banded per matrix: per block step a diagonal kernel (factor + block inverse), a panel kernel
-// (A_ib,kb <- A_ib,kb W^T on MFMA) and a trailing-update kernel (A_IJ -= P_I P_J^T on MFMA).
+// or banded per matrix: diagonal blocks (factor + block inverse W), left-looking panel steps
+// (A_ib,kb <- (A_ib,kb - earlier blocks) W^T) and trailing updates (A_IJ -= P_I P_J^T), products on MFMA.
 // Matrices with fewer blocks skip the step; the upper triangle is never written.
 // Restates Cholesky_dcmp_packed (pixelgrid.cpp:17071-17105) blockwise: a pivot of a row < n that
 // is not positive (negative, zero or NaN) sets *status and the factorization continues with
@@ -1696,9 +1700,9 @@ __device__ __forceinline__ void mma64(T (*As)[LDT], T (*Bs)[LDT], typename Mfma1
     mma64_add<T>(As, Bs, acc);
 }
 
-// C (64x64 at row pitch ldc) = acc (mode 0), C -= acc (mode 1), lower triangle only (mode 2)
+// C (64x64 at row pitch ldc) = acc
 template <typename T>
-__device__ __forceinline__ void store64(T* C, int ldc, const typename Mfma16<T>::acc_t acc[2][2], int mode)
+__device__ __forceinline__ void store64(T* C, int ldc, const typename Mfma16<T>::acc_t acc[2][2])
 {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int wr = w >> 1, wc = w & 1;
@@ -1710,14 +1714,12 @@ __device__ __forceinline__ void store64(T* C, int ldc, const typename Mfma16<T>:
             for (int v = 0; v < 4; v++) {
                 const int rr = wr * 32 + a * 16 + Mfma16<T>::row(lane, v);
                 const int cc = wc * 32 + c * 16 + (lane & 15);
-                T* d = C + (size_t)rr * ldc + cc;
-                if (mode == 0) *d = acc[a][c][v];
-                else if (mode == 1 || cc <= rr) *d -= acc[a][c][v];
+                C[(size_t)rr * ldc + cc] = acc[a][c][v];
             }
 }
 
 // the 16 C values of a lane (store64's layout), loaded before the staging barrier so their latency
-// overlaps the operand loads; store64c then writes C - acc (mode 1) or its lower triangle (mode 2)
+// overlaps the operand loads
 template <typename T>
 __device__ __forceinline__ void load64c(const T* C, int ldc, T (&cv)[16])
 {
@@ -1735,301 +1737,9 @@ __device__ __forceinline__ void load64c(const T* C, int ldc, T (&cv)[16])
             }
 }
 
-template <typename T>
-__device__ __forceinline__ void store64c(T* C, int ldc, const typename Mfma16<T>::acc_t acc[2][2], const T (&cv)[16], int mode)
-{
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int wr = w >> 1, wc = w & 1;
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int rr = wr * 32 + a * 16 + Mfma16<T>::row(lane, v);
-                const int cc = wc * 32 + c * 16 + (lane & 15);
-                if (mode == 1 || cc <= rr) C[(size_t)rr * ldc + cc] = cv[(a * 2 + c) * 4 + v] - acc[a][c][v];
-            }
-}
-
-#define MM_LDS (2 * TS * LDT)
-template <typename T>
-__device__ void chol_panel_body(const MatDesc& D, int kb, int ib, double* raw)
-{
-    T(*As)[LDT] = (T(*)[LDT])raw;
-    T(*Bs)[LDT] = (T(*)[LDT])((T*)raw + TS * LDT);
-    int ld;
-    T* blk = tile_ptr<T>(D, ib, kb, ld);
-    const T* W = (const T*)D.W + (size_t)kb * TS * TS;
-    stage64<T>(blk, ld, As);
-    stage64<T>(W, TS, Bs);
-    __syncthreads();
-    typename Mfma16<T>::acc_t acc[2][2];
-    mma64<T>(As, Bs, acc);  // C(i,j) = sum_q A_ib[i][q] W[j][q]
-    store64<T>(blk, ld, acc, 0);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_chol_panel_m(const MatDesc* mats, int kb)
-{
-    __shared__ T raw[MM_LDS];
-    const MatDesc D = mats[blockIdx.y];
-    if (kb >= D.nb) return;
-    const int ib = kb + 1 + blockIdx.x;
-    if (ib > band_last(D, kb)) return;
-    chol_panel_body<T>(D, kb, ib, (double*)raw);
-}
-
-// trailing update A_IJ -= P_I P_J^T for one element type (matrices of one launch share it)
-template <typename T>
-__global__ void __launch_bounds__(256) k_chol_update_m(const MatDesc* mats, int kb)
-{
-    __shared__ T As[TS][LDT];
-    __shared__ T Bs[TS][LDT];
-    const MatDesc D = mats[blockIdx.y];
-    if (kb >= D.nb) return;
-    const int rest = band_last(D, kb) - kb;
-    int I, J;
-    if (!syrk_tile(rest, I, J)) return;  // XCD-aware super-tile order: neighbours share panel blocks in L2
-    I += kb + 1;
-    J += kb + 1;
-    int lda, ldb, ldc;
-    const T* Pa = tile_ptr<T>(D, I, kb, lda);
-    const T* Pb = tile_ptr<T>(D, J, kb, ldb);
-    T* C = tile_ptr<T>(D, I, J, ldc);
-    T cv[16];
-    load64c<T>(C, ldc, cv);
-    stage64<T>(Pa, lda, As);
-    stage64<T>(Pb, ldb, Bs);
-    __syncthreads();
-    typename Mfma16<T>::acc_t acc[2][2];
-    mma64<T>(As, Bs, acc);
-    store64c<T>(C, ldc, acc, cv, I == J ? 2 : 1);
-}
-
-// rank-64 update from column block kb of the tiles (I, J), kb < J < kend, J <= I < nb: the
-// columns of the current 256-wide panel that are still to be factored (dense matrices only)
-template <typename T>
-__global__ void __launch_bounds__(256) k_chol_upanel_m(const MatDesc* mats, int kb, int kend)
-{
-    __shared__ T As[TS][LDT];
-    __shared__ T Bs[TS][LDT];
-    const MatDesc D = mats[blockIdx.y];
-    if (kb >= D.nb) return;
-    const int je = min(kend, D.nb);
-    int t = blockIdx.x, I = -1, J = -1;
-    for (int j = kb + 1; j < je; j++) {
-        const int cnt = D.nb - j;
-        if (t < cnt) {
-            J = j;
-            I = j + t;
-            break;
-        }
-        t -= cnt;
-    }
-    if (J < 0) return;
-    int lda, ldb, ldc;
-    const T* Pa = tile_ptr<T>(D, I, kb, lda);
-    const T* Pb = tile_ptr<T>(D, J, kb, ldb);
-    T* C = tile_ptr<T>(D, I, J, ldc);
-    T cv[16];
-    load64c<T>(C, ldc, cv);
-    stage64<T>(Pa, lda, As);
-    stage64<T>(Pb, ldb, Bs);
-    __syncthreads();
-    typename Mfma16<T>::acc_t acc[2][2];
-    mma64<T>(As, Bs, acc);
-    store64c<T>(C, ldc, acc, cv, I == J ? 2 : 1);
-}
-
-// Left-looking step of a 256-wide panel (columns k0 .. kend-1, dense matrices): column block kb.
-// Workgroup x takes row block ib = kb + 1 + x and forms
-//   A_ib,kb - sum_{k0 <= k' < kb} L_ib,k' L_kb,k'^T  (the earlier columns of the panel, summed in
-//   the MFMA accumulators while the block waits in registers),  L_ib,kb = that times W_kb^T,
-// so each block is read and written once per panel column.  The workgroup of ib = kb + 1 then
-// brings the next diagonal block up to date for the diagonal kernel, when it lies in the panel:
-//   A_ib,ib -= sum_{k0 <= k' <= kb} L_ib,k' L_ib,k'^T  (lower half stored).
-template <typename T>
-__global__ void __launch_bounds__(256) k_chol_lpanel_m(const MatDesc* mats, int kb, int k0, int kend)
-{
-    __shared__ T As[TS][LDT];
-    __shared__ T Bs[TS][LDT];
-    typedef typename Mfma16<T>::acc_t Acc;
-    const MatDesc D = mats[blockIdx.y];
-    if (kb >= D.nb) return;
-    const int ib = kb + 1 + blockIdx.x;
-    if (ib > band_last(D, kb)) return;
-    int ld, lp;
-    T* blk = tile_ptr<T>(D, ib, kb, ld);
-    // the part that starts at column 0 reads its blocks from F as formed (A0), when the matrix has
-    // it: each is read there once and written to A
-    const bool first = (k0 == 0 && D.A0);
-    T cv[16];
-    load64c<T>(first ? (const T*)D.A0 + (blk - (T*)D.A) : blk, ld, cv);
-    Acc acc[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int c = 0; c < 2; c++) acc[a][c] = (Acc){0, 0, 0, 0};
-    for (int kp = k0; kp < kb; kp++) {
-        const T* Pa = tile_ptr<T>(D, ib, kp, lp);
-        const T* Pb = tile_ptr<T>(D, kb, kp, lp);
-        __syncthreads();
-        stage64<T>(Pa, lp, As);
-        stage64<T>(Pb, lp, Bs);
-        __syncthreads();
-        mma64_add<T>(As, Bs, acc);
-    }
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) acc[a][c][v] = cv[(a * 2 + c) * 4 + v] - acc[a][c][v];
-    __syncthreads();
-    store64<T>(&As[0][0], LDT, acc, 0);
-    stage64<T>((const T*)D.W + (size_t)kb * TS * TS, TS, Bs);
-    __syncthreads();
-    mma64<T>(As, Bs, acc);  // L_ib,kb(i, j) = sum_q A'(i, q) W_kb(j, q)
-    store64<T>(blk, ld, acc, 0);
-    if (ib != kb + 1 || ib >= kend) return;
-    T* dg = tile_ptr<T>(D, ib, ib, ld);
-    load64c<T>(first ? (const T*)D.A0 + (dg - (T*)D.A) : dg, ld, cv);
-    __syncthreads();
-    store64<T>(&As[0][0], LDT, acc, 0);
-    __syncthreads();
-    mma64<T>(As, As, acc);
-    for (int kp = k0; kp < kb; kp++) {
-        const T* Pa = tile_ptr<T>(D, ib, kp, lp);
-        __syncthreads();
-        stage64<T>(Pa, lp, As);
-        __syncthreads();
-        mma64_add<T>(As, As, acc);
-    }
-    store64c<T>(dg, ld, acc, cv, 2);
-}
-
-// acc += As(rows of quadrant wr) * Bs(rows of quadrant wc)^T over the 64 staged columns.  Lane group
-// g = lane/16 reads VW consecutive k of its row with one LDS vector read; MFMA s of the group takes
-// component s, so the VW MFMAs of a step sum k = kk + VW*g + s over all 4*VW values of the step.
-template <typename T>
-__device__ __forceinline__ void trail_mma(T (*As)[LDT], T (*Bs)[LDT], typename Mfma16<T>::acc_t (&acc)[4][4])
-{
-    typedef typename Mfma16<T>::vec_t V;
-    constexpr int VW = sizeof(V) / sizeof(T);
-    typedef T P __attribute__((ext_vector_type(VW)));
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int wr = w >> 1, wc = w & 1;
-#pragma unroll 1
-    for (int kk = 0; kk < TS; kk += 4 * VW) {
-        const int kq = kk + VW * (lane >> 4);
-        P av[4], bv[4];
-#pragma unroll
-        for (int a = 0; a < 4; a++) av[a] = *(const P*)&As[wr * 64 + a * 16 + (lane & 15)][kq];
-#pragma unroll
-        for (int c = 0; c < 4; c++) bv[c] = *(const P*)&Bs[wc * 64 + c * 16 + (lane & 15)][kq];
-#pragma unroll
-        for (int s2 = 0; s2 < VW; s2++)
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int c = 0; c < 4; c++) acc[a][c] = Mfma16<T>::op(av[a][s2], bv[c][s2], acc[a][c]);
-    }
-}
-
-// Trailing update after a 256-wide panel: C(I, J) -= sum over the panel's nq column blocks of
-// L(I, q) L(J, q)^T, on 128 x 128 tiles of the trailing matrix (first row block k0 + nq, XCD-aware
-// tile order).  Wave (wr, wc) owns the 64 x 64 quadrant (wr, wc): 4 x 4 MFMA tiles of 16 x 16.
-#define TT 128
-// Two 128 x 68 staging tiles per WG (70 KB in FP32) allow two WGs per CU, so two waves per SIMD
-// is all the occupancy this kernel gets: the register budget is sized for that.
-template <typename T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 1 : 2, sizeof(T) == 8 ? 1 : 2)))
-k_chol_trail_m(const MatDesc* mats, int k0, int nq)
-{
-    extern __shared__ double trail_raw[];
-    T(*As)[LDT] = (T(*)[LDT])trail_raw;
-    T(*Bs)[LDT] = (T(*)[LDT])((T*)trail_raw + TT * LDT);
-    const MatDesc D = mats[blockIdx.y];
-    const int r0b = k0 + nq;
-    if (r0b >= D.nb) return;
-    const int nt = (D.nb - r0b) / 2;
-    int I2, J2;
-    if (!syrk_tile(nt, I2, J2)) return;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int wr = w >> 1, wc = w & 1;
-    const long long ld = D.ld;
-    T* A = (T*)D.A;
-    const long long rI = (long long)(r0b + 2 * I2) * TS, rJ = (long long)(r0b + 2 * J2) * TS;
-    typename Mfma16<T>::acc_t acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) acc[a][c] = (typename Mfma16<T>::acc_t){0, 0, 0, 0};
-    typedef typename Mfma16<T>::vec_t V;
-    constexpr int VW = sizeof(V) / sizeof(T);
-    constexpr int NPF = (TT * TS) / (256 * VW);  // pieces per thread and matrix
-    typedef T P __attribute__((ext_vector_type(VW)));
-    P pa[NPF], pb[NPF];
-    T cv[64];  // the C tile values of this lane (loaded during the last block)
-    // the next column block is loaded into registers while the current one is multiplied (FP64: one
-    // workgroup per CU for its 139 KB of LDS, so the registers are there)
-#define TRAIL_LOAD(q)                                                    \
-    {                                                                    \
-        const long long c0 = (long long)(k0 + (q)) * TS;                 \
-        _Pragma("unroll") for (int h = 0; h < NPF; h++)                  \
-        {                                                                \
-            const int e = (tid + 256 * h) * VW;                          \
-            const int i = e >> 6, k = e & 63;                            \
-            pa[h] = *(const P*)&A[(rI + i) * ld + c0 + k];               \
-            pb[h] = *(const P*)&A[(rJ + i) * ld + c0 + k];               \
-        }                                                                \
-    }
-    {
-        TRAIL_LOAD(0);
-        for (int q = 0; q < nq; q++) {
-            __syncthreads();
-#pragma unroll
-            for (int h = 0; h < NPF; h++) {
-                const int e = (tid + 256 * h) * VW;
-                const int i = e >> 6, k = e & 63;
-                *(P*)&As[i][k] = pa[h];
-                *(P*)&Bs[i][k] = pb[h];
-            }
-            __syncthreads();
-            if (q + 1 == nq) break;  // the last block is multiplied below, with the C tile loads
-            TRAIL_LOAD(q + 1);
-            trail_mma<T>(As, Bs, acc);
-        }
-#pragma unroll
-        for (int a = 0; a < 4; a++)
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int rr = wr * 64 + a * 16 + Mfma16<T>::row(lane, v);
-                    const int cc = wc * 64 + c * 16 + (lane & 15);
-                    cv[(a * 4 + c) * 4 + v] = A[(rI + rr) * ld + rJ + cc];
-                }
-        trail_mma<T>(As, Bs, acc);
-    }
-    const bool diag = (I2 == J2);
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int rr = wr * 64 + a * 16 + Mfma16<T>::row(lane, v);
-                const int cc = wc * 64 + c * 16 + (lane & 15);
-                T* d = &A[(rI + rr) * ld + rJ + cc];
-                const T old = cv[(a * 4 + c) * 4 + v];
-                if (!diag || cc <= rr) *d = old - acc[a][c][v];
-            }
-}
-#undef TRAIL_LOAD
-
-// FP32 matrices (mixed path): the same trailing update with the panel operands split x = hi + lo
+#define TT 128  // tile side of the trailing updates
+// FP32 matrices (mixed path): the trailing update C(I, J) -= sum over the panel's column blocks of
+// L(I, q) L(J, q)^T on 128 x 128 tiles, with the panel operands split x = hi + lo
 // into BF16 while they are staged (hi = bf16(x), lo = bf16(x - hi): 2^-17 of each entry, with the
 // hardware round-to-nearest conversion) and all four products hi*hi + hi*lo + lo*hi + lo*lo on
 // v_mfma_f32_16x16x32_bf16, accumulated in FP32.  The accumulators start from the C tile and the A
@@ -2189,7 +1899,7 @@ k_chol_trail_bf16(const MatDesc* mats, int k0, int nq, int ncolt, int fdiag)
     }
 }
 
-// The left-looking panel step for FP32 matrices (k_chol_lpanel_m's schedule and operands) with the
+// The left-looking panel step for FP32 matrices (the FP64 one's schedule) with the
 // products on v_mfma_f32_16x16x32_bf16: every operand is split x = hi + lo into BF16 as it is
 // staged (as in k_chol_trail_bf16) and the four products hi*hi + hi*lo + lo*hi + lo*lo are summed
 // in FP32 (1.9 ms faster than FP32 MFMA per batch of 256 3712 x 3712 matrices; |delta lnE| against
@@ -2381,87 +2091,223 @@ __device__ __forceinline__ void chol_diag_f32_4w(const MatDesc& D, int kb, float
     for (int j = 0; j < 16; j++) W[(16 * w + j) * TS + r] = x[j];
 }
 
-// The FP64 diagonal block by the same four-wave panel scheme: d = sqrt|p|, l = a / d; row q of L^-1
-// divided by L(q, q), its updates applied in row order (the left-looking substitution's fused
-// multiply-adds in the same order, so the same bits as that form).  LDS: Lt
-// 64 x 64, X 2 x 16 x 64 (panel p's rows in X[p & 1]: the barrier after panel p + 1 orders their
-// readers before panel p + 2 rewrites them).
-__device__ __forceinline__ void chol_diag_f64_4w(const MatDesc& D, int kb, double* tile, int ld, double (&a)[16],
-                                                 double (*Lt)[TS], double (*X)[16][TS])
+// 1 / sqrt(p) of a positive FP64 p: the hardware estimate (about 2^-23) and one third-order step
+// (r e (1/2 + 3/8 e) with e = 1 - p r^2 leaves an error of order e^3, below the last place)
+__device__ __forceinline__ double rsqrt_f64(double p)
+{
+    const double r = __builtin_amdgcn_rsq(p);
+    const double e = fma(-(p * r), r, 1.0);
+    return fma(r * e, fma(0.375, e, 0.5), r);
+}
+// a / d for r = 1 / d to within an ulp: one correction from the exact remainder
+__device__ __forceinline__ double div_r(double a, double d, double r)
+{
+    const double q = a * r;
+    return fma(fma(-q, d, a), r, q);
+}
+
+// 1 / p of an FP64 p > 0 likewise (e = 1 - p r, r (1 + e + e^2))
+__device__ __forceinline__ double rcp_f64(double p)
+{
+    const double r = __builtin_amdgcn_rcp(p);
+    const double e = fma(-p, r, 1.0);
+    return fma(r * e, 1.0 + e, r);
+}
+
+// lane C of each 16-lane row in all of the row's lanes
+template <int C>
+__device__ __forceinline__ double row_bcast_f64(double v)
+{
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, 0x150 + C, 0xf, 0xf, false);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), 0x150 + C, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+// x (row m of four columns of the identity) through the elimination's steps c = 0 .. 14
+template <int... C>
+__device__ __forceinline__ void z_steps(double (&x)[4], const double (&mc)[15], std::integer_sequence<int, C...>)
+{
+    auto step = [&](auto c) {
+        constexpr int cc = decltype(c)::value;
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = fma(-mc[cc], row_bcast_f64<cc>(x[j]), x[j]);
+    };
+    (step(std::integral_constant<int, C>()), ...);
+}
+
+// The FP64 diagonal block and its inverse by four waves, in 16 x 16 blocks.  It is the serial chain of
+// every FP64 factorization, so it is arranged for latency (34 us a launch on one
+// matrix as rank-1 updates with a square root and a division a column, now 16):
+//   * wave t factors panel t (columns 16 t .. 16 t + 15), one row per lane, without square roots
+//     (A = M P M^T, M unit lower): a column's chain is its pivot's reciprocal, one product and the next
+//     pivot's update, with the next two columns' entries broadcast by readlane; the other columns take
+//     theirs from LDS a column later, and the sixteen 1 / sqrt(p) are formed at once afterwards;
+//   * the waves after t then update their panels' blocks with v_mfma_f64_16x16x4f64 (operands M P and
+//     M), held in the accumulator layout until their turn;
+//   * wave j owns column block j of M^-1: Z_jj by eliminating the identity while wave j + 1 factors,
+//     then Z_ij = -Z_ii sum_k M_ik Z_kj on MFMA as the Z_ii appear (an accumulator is a B operand as it
+//     lies); L^-1 = P^-1/2 M^-1 and L = M P^1/2 are scaled on the way out.
+// Phases 0 .. 4 end with a barrier; in phase t wave t factors, wave t - 1 forms Z_(t-1)(t-1), the waves
+// before finish row t - 2 and sum for row t - 1.  acc[i] holds rows 16 i .. of the wave's 16 columns
+// (i >= w; the accumulator layout).  LDS: DGL doubles.
+#define DGP 74                      // row pitch: rows and columns of 16 spread over the banks, pairs aligned
+#define DGL (2 * TS * DGP + 2 * TS) // Mt[c][r] = M(r, c), Z by rows, the pivots, their 1 / sqrt
+__device__ __forceinline__ void chol_diag_f64_4w(const MatDesc& D, int kb, double* tile, int ld, double4_t (&acc)[4], double* sm)
 {
     typedef double T;
-    const int r = threadIdx.x & 63, w = threadIdx.x >> 6;
+    T(*Z)[DGP] = (T(*)[DGP])sm;
+    T(*Mt)[DGP] = (T(*)[DGP])(sm + TS * DGP);
+    T* const Pv = sm + 2 * TS * DGP;
+    T* const Rs = Pv + TS;
+    const int r = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m = r & 15, g = r >> 4;
+    const int w16 = 16 * w;
     const long long base = (long long)kb * TS;
-    bool bad = false;
+    T* const W = (T*)D.W + (size_t)kb * TS * TS;
+    // panel t's update of the blocks i >= I0 (= w, known to the compiler: no branch between the MFMAs)
+    auto update = [&](int t, auto I0) {
+        constexpr int i0 = decltype(I0)::value;
+        T b[4], av[4][4];
 #pragma unroll
-    for (int p = 0; p < 4; p++) {
-        if (w == p) {
+        for (int s = 0; s < 4; s++) {
+            const int c = 16 * t + 4 * s + g;
+            b[s] = Mt[c][w16 + m];
+            const T pc = -Pv[c];
 #pragma unroll
-            for (int cc = 0; cc < 16; cc++) {
-                const int c = 16 * p + cc;
-                const T piv = readlane_f64(a[cc], c);
-                bad |= (!(piv > 0) && base + c < D.n);  // negative, zero or NaN pivot
-                const T d = sqrt(fabs(piv));
-                const T l = (r > c) ? a[cc] / d : d;
-                a[cc] = l;
-                Lt[c][r] = l;
-                wave_lds_sync();
-#pragma unroll
-                for (int j = cc + 1; j < 16; j++) a[j] = fma(-l, Lt[c][16 * p + j], a[j]);
-            }
+            for (int i = i0; i < 4; i++) av[s][i] = Mt[c][16 * i + m] * pc;
         }
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = i0; i < 4; i++) acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s][i], b[s], acc[i], 0, 0, 0);
+    };
+#pragma unroll 1
+    for (int t = 0; t < w; t++) {
         __syncthreads();
-        if (w > p) {
+        if (w == 1) update(t, std::integral_constant<int, 1>());
+        else if (w == 2) update(t, std::integral_constant<int, 2>());
+        else update(t, std::integral_constant<int, 3>());
+    }
+    // ---- phase w: the panel, one row per lane ----
+    T a[16];
 #pragma unroll
-            for (int cc = 0; cc < 16; cc++) {
-                const int c = 16 * p + cc;
-                const T l = Lt[c][r];
+    for (int i = 0; i < 4; i++)
 #pragma unroll
-                for (int j = 0; j < 16; j++) a[j] = fma(-l, Lt[c][16 * w + j], a[j]);
+        for (int v = 0; v < 4; v++) Mt[w16 + m][16 * i + 4 * v + g] = i >= w ? acc[i][v] : (T)0;
+    wave_lds_sync();
+#pragma unroll
+    for (int j = 0; j < 16; j++) a[j] = Mt[w16 + j][r];
+    wave_lds_sync();
+    {
+        T p = readlane_f64(a[0], w16);
+        T ap = (T)0, myp = (T)1;  // the previous column; the lane's own pivot
+        double2_t vp[8];          // its multipliers of columns >= c + 2, still to be applied
+        int mo;                   // &Mt[w16][w16] in a vector register: every broadcast read is an immediate offset away
+        asm("v_mov_b32 %0, %1" : "=v"(mo) : "s"((TS + w16) * DGP + w16));
+#pragma unroll
+        for (int c = 0; c < 16; c++) {
+            const T rp = rcp_f64(fabs(p));
+            myp = (r == w16 + c) ? a[c] : myp;
+            const T v = a[c] * rp;
+            Mt[w16 + c][r] = v;
+            if (c < 15) {
+                a[c + 1] = fma(-a[c], readlane_f64(v, w16 + c + 1), a[c + 1]);
+                p = readlane_f64(a[c + 1], w16 + c + 1);
+            }
+            if (c < 14) a[c + 2] = fma(-a[c], readlane_f64(v, w16 + c + 2), a[c + 2]);
+#pragma unroll
+            for (int j = c + 2; j < 16; j++)
+                if (c > 0) a[j] = fma(-ap, vp[j >> 1][j & 1], a[j]);
+            wave_lds_sync();
+#pragma unroll
+            for (int j = (c + 3) / 2; j < 8; j++) vp[j] = *(const double2_t*)&sm[mo + c * DGP + 2 * j];
+            ap = a[c];
+        }
+        if (g == w) Pv[r] = myp;
+    }
+    __syncthreads();
+    // ---- phase w + 1: Z_ww by the same elimination of the identity ----
+    const T pv = Pv[w16 + m];  // pivot of the lane's row within the block, its square root and inverse
+    const T pa = fabs(pv);
+    const T rs = rsqrt_f64(pa);
+    T dg = pa * rs;
+    dg = fma(fma(-dg, dg, pa), 0.5 * rs, dg);
+    const bool own = g == w;  // lanes of the panel's own rows
+    {
+        // lane (m, g): row m, columns 4 g .. 4 g + 3; row c's entries come from lane c of the 16-lane row
+        T x[4], mc[15];
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = (m == 4 * g + j) ? (T)1 : (T)0;
+#pragma unroll
+        for (int c = 0; c < 15; c++) mc[c] = m > c ? Mt[w16 + c][w16 + m] : (T)0;
+        z_steps(x, mc, std::make_integer_sequence<int, 15>());
+        if (g == 0) Rs[w16 + m] = rs;
+#pragma unroll
+        for (int j = 0; j < 4; j++) Z[w16 + m][w16 + 4 * g + j] = x[j];
+#pragma unroll
+        for (int j = 0; j < 4; j += 2)
+            *(double2_t*)&W[(w16 + m) * TS + w16 + 4 * g + j] = (double2_t){x[j] * rs, x[j + 1] * rs};
+    }
+    // L's panel (M P^1/2 below the diagonal) and what lies above it in L^-1
+    auto finish = [&]() {
+#pragma unroll
+        for (int c = 0; c < 16; c++) a[c] = (r == w16 + c) ? dg : div_r(a[c], readlane_f64(dg, c), readlane_f64(rs, c));
+#pragma unroll
+        for (int j = 0; j < 16; j += 2) {
+            const int q = w16 + j;
+            T* dst = tile + (size_t)r * ld + q;
+            if (q + 1 <= r) {
+                *(double2_t*)dst = (double2_t){a[j], a[j + 1]};
+            } else if (q <= r) {
+                dst[0] = a[j];
             }
         }
-    }
-    if (r == 0 && bad) atomicOr(D.status, 1);
+        if (g < w) {
 #pragma unroll
-    for (int j = 0; j < 16; j += 2) {
-        const int q = 16 * w + j;
-        T* dst = tile + (size_t)r * ld + q;
-        if (q + 1 <= r) {
-            *(double2*)dst = make_double2(a[j], a[j + 1]);
-        } else if (q <= r) {
-            dst[0] = a[j];
+            for (int j = 0; j < 16; j += 2) *(double2_t*)&W[r * TS + w16 + j] = (double2_t){0, 0};
         }
-    }
-    if (w == 0) ((T*)D.diag)[base + r] = Lt[r][r];
-    T x[16];
+        if (own) {
+            ((T*)D.diag)[base + r] = dg;
+            if (!(pv > 0) && base + r < D.n) atomicOr(D.status, 1);  // negative, zero or NaN pivot
+        }
+    };
+    // ---- phases w + 2 .. 5: the sum of row t - 1, and row t - 2 of the sum formed a phase earlier ----
+    double4_t S = {0, 0, 0, 0};
+#pragma unroll 1
+    for (int t = w + 1; t <= 5; t++) {
+        if (t - 2 > w) {  // Z_iw = -Z_ii S, i = t - 2
+            const int i = t - 2;
+            double4_t o = {0, 0, 0, 0};
+            T av[4];
 #pragma unroll
-    for (int j = 0; j < 16; j++) x[j] = (16 * w + j == r) ? (T)1 : (T)0;
+            for (int s = 0; s < 4; s++) av[s] = -Z[16 * i + m][16 * i + 4 * s + g];
 #pragma unroll
-    for (int p = 0; p < 4; p++) {
-        if (w == p) {
+            for (int s = 0; s < 4; s++) o = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s], S[s], o, 0, 0, 0);
 #pragma unroll
-            for (int qq = 0; qq < 16; qq++) {
-                const int q = 16 * p + qq;
-                x[qq] = (r <= q) ? x[qq] / Lt[q][q] : (T)0;
-                X[p & 1][qq][r] = x[qq];
+            for (int v = 0; v < 4; v++) {
+                Z[16 * i + 4 * v + g][w16 + m] = o[v];
+                W[(16 * i + 4 * v + g) * TS + w16 + m] = o[v] * Rs[16 * i + 4 * v + g];
+            }
+            wave_lds_sync();
+        }
+        if (t - 1 > w && t <= 4) {  // S_iw = sum_(k = w)^(i - 1) M_ik Z_kw, i = t - 1
+            const int i = t - 1;
+            S = (double4_t){0, 0, 0, 0};
+#pragma unroll 1
+            for (int k = w; k < i; k++) {
+                T av[4], bv[4];
 #pragma unroll
-                for (int j = qq + 1; j < 16; j++) x[j] = fma(-Lt[q][16 * p + j], x[qq], x[j]);
+                for (int s = 0; s < 4; s++) {
+                    av[s] = Mt[16 * k + 4 * s + g][16 * i + m];
+                    bv[s] = Z[16 * k + 4 * s + g][w16 + m];
+                }
+#pragma unroll
+                for (int s = 0; s < 4; s++) S = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s], bv[s], S, 0, 0, 0);
             }
         }
-        __syncthreads();
-        if (w > p) {
-#pragma unroll
-            for (int qq = 0; qq < 16; qq++) {
-                const int q = 16 * p + qq;
-                const T xq = X[p & 1][qq][r];
-#pragma unroll
-                for (int j = 0; j < 16; j++) x[j] = fma(-Lt[q][16 * w + j], xq, x[j]);
-            }
-        }
+        if (t == w + 2) finish();  // (the last wave's comes in phase 5)
+        if (t < 5) __syncthreads();
     }
-    T* W = (T*)D.W + (size_t)kb * TS * TS;
-#pragma unroll
-    for (int j = 0; j < 16; j++) W[(16 * w + j) * TS + r] = x[j];
 }
 
 // one diagonal block per matrix (blockIdx.y), four waves; FP32 blocks of the first column read F as
@@ -2475,27 +2321,27 @@ __global__ void __launch_bounds__(256) k_chol_diag4_m(const MatDesc* mats, int k
     T* tile = tile_ptr<T>(D, kb, kb, ld);
     const T* src = (sizeof(T) == 4 && kb == 0 && D.A0) ? (const T*)D.A0 + (tile - (T*)D.A) : tile;
     const int r = threadIdx.x & 63, w = threadIdx.x >> 6;
-    typedef typename Mfma16<T>::vec_t V;
-    constexpr int VW = sizeof(V) / sizeof(T);
-    T a[16];
-#pragma unroll
-    for (int j = 0; j < 16; j += VW) {
-        const V v = *(const V*)&src[(size_t)r * ld + 16 * w + j];
-        a[j] = v.x;
-        a[j + 1] = v.y;
-        if constexpr (VW == 4) {
-            a[j + 2] = v.z;
-            a[j + 3] = v.w;
-        }
-    }
     if constexpr (sizeof(T) == 8) {
-        __shared__ double Lt[TS][TS];
-        __shared__ double X[2][16][TS];
-        chol_diag_f64_4w(D, kb, tile, ld, a, Lt, X);
+        __shared__ __align__(16) double sm[DGL];
+        double4_t acc[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) acc[i][v] = i >= w ? src[(size_t)(16 * i + 4 * v + (r >> 4)) * ld + 16 * w + (r & 15)] : 0.0;
+        chol_diag_f64_4w(D, kb, tile, ld, acc, sm);
     } else {
         __shared__ __align__(16) float Lt[TS][TS];
         __shared__ float X[TS][TS];
         __shared__ float Rd[TS];
+        float a[16];
+#pragma unroll
+        for (int j = 0; j < 16; j += 4) {
+            const float4_t v = *(const float4_t*)&src[(size_t)r * ld + 16 * w + j];
+            a[j] = v.x;
+            a[j + 1] = v.y;
+            a[j + 2] = v.z;
+            a[j + 3] = v.w;
+        }
         chol_diag_f32_4w(D, kb, tile, ld, a, Lt, X, Rd);
     }
 }
@@ -2562,7 +2408,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
 #pragma unroll
         for (int c = 0; c < 2; c++) acc[a][c] = (float4_t){0, 0, 0, 0};
     mma64_bf16(Ah, Al, Bh, Bl, acc);  // L_ib,kb(i, j) = sum_q A'(i, q) W_kb(j, q)
-    store64<T>(blk, ld, acc, 0);
+    store64<T>(blk, ld, acc);
     if (ib != kb + 1 || ib >= kend) return;
     T* dg = tile_ptr<T>(D, ib, ib, ld);
     load64c<T>(first ? (const T*)D.A0 + (dg - (T*)D.A) : dg, ld, cv);
@@ -2609,92 +2455,261 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k
     }
 }
 
-template <typename T>
-static void chol_step(hipStream_t s, const MatDesc* mats, int nmat, int kb, int rest)
+// acc += A B^T over nst stages of 16 k, 64 rows of A and of B: wave (wr, wc) of four holds 32 rows of each
+// as 2 x 2 accumulators.  Rows lie lda (ldb) apart; 64-column block q of a row starts q * ba
+// (bb) after the first (64 in a dense matrix, -4096 along a banded row).  Operands go through two LDS
+// buffers, one barrier a stage, loaded a stage ahead; rows 144 bytes apart put the 16 rows of an operand
+// read on distinct 16-byte slots.
+#define TFP 18
+__device__ __forceinline__ void gemm_f64(const double* A, size_t lda, long long ba, const double* B, size_t ldb, long long bb, int nst,
+                                         double* lds, double4_t (&acc)[2][2])
 {
-    hipLaunchKernelGGL(k_chol_diag4_m<T>, dim3(1, nmat), dim3(256), 0, s, mats, kb);
-    if (rest > 0) {  // rest: the widest trailing extent of any matrix in the launch
-        hipLaunchKernelGGL(k_chol_panel_m<T>, dim3(rest, nmat), dim3(256), 0, s, mats, kb);
-        hipLaunchKernelGGL(k_chol_update_m<T>, dim3(syrk_grid(rest), nmat), dim3(256), 0, s, mats, kb);
-    }
-}
-
-// one column block after another of the panel [k0, kend): the diagonal kernel, then the panel kernel
-template <typename T>
-static void chol_subpanel(hipStream_t s, const MatDesc* mats, int nmat, int max_nb, int k0, int kend, bool left,
-                          bool first_done = false)
-{
-    for (int kb = k0; kb < kend && kb < max_nb; kb++) {
-        const int rest = max_nb - kb - 1;
-        const bool f32 = sizeof(T) == 4;
-        // FP32 left-looking parts: the panel kernel of column block kb - 1 factored block kb, and
-        // the update before the part factored block k0 (first_done)
-        if (!(left && f32 && (kb > k0 || first_done))) hipLaunchKernelGGL(k_chol_diag4_m<T>, dim3(1, nmat), dim3(256), 0, s, mats, kb);
-        if (rest <= 0) continue;
-        if (left) {
-            if (f32)
-                hipLaunchKernelGGL(k_chol_lpanel_bf16, dim3(nmat, rest), dim3(256), 0, s, mats, kb, k0, kend);
-            else
-                hipLaunchKernelGGL(k_chol_lpanel_m<T>, dim3(rest, nmat), dim3(256), 0, s, mats, kb, k0, kend);
-            continue;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int wr = w >> 1, wc = w & 1;
+    // piece h of a thread: row (tid >> 3) + 32 h, columns 2 (tid & 7) and the next of the stage
+    const double* const pA = A + (tid >> 3) * lda + 2 * (tid & 7);
+    const double* const pB = B + (tid >> 3) * ldb + 2 * (tid & 7);
+    double* const st0 = lds + (tid >> 3) * TFP + 2 * (tid & 7);
+    const double* const a0 = lds + (wr * 32 + (lane & 15)) * TFP + 2 * (lane >> 4);
+    const double* const b0 = lds + (TS + wc * 32 + (lane & 15)) * TFP + 2 * (lane >> 4);
+    double2_t ra[2], rb[2];
+    auto load = [&](int st) {
+        const long long oa = (st >> 2) * ba + (st & 3) * 16, ob = (st >> 2) * bb + (st & 3) * 16;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            ra[h] = *(const double2_t*)(pA + (size_t)(32 * h) * lda + oa);
+            rb[h] = *(const double2_t*)(pB + (size_t)(32 * h) * ldb + ob);
         }
-        hipLaunchKernelGGL(k_chol_panel_m<T>, dim3(rest, nmat), dim3(256), 0, s, mats, kb);
-        int cnt = 0;
-        for (int j = kb + 1; j < kend && j < max_nb; j++) cnt += max_nb - j;
-        if (cnt > 0) hipLaunchKernelGGL(k_chol_upanel_m<T>, dim3(cnt, nmat), dim3(256), 0, s, mats, kb, kend);
+    };
+    auto stage = [&](int buf) {
+        double* const d = st0 + buf * 2 * TS * TFP;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            *(double2_t*)(d + 32 * h * TFP) = ra[h];
+            *(double2_t*)(d + (TS + 32 * h) * TFP) = rb[h];
+        }
+    };
+    load(0);
+    stage(0);
+    for (int st = 0; st < nst; st++) {
+        __syncthreads();  // stage st is in its buffer, and the other buffer's readers are done
+        if (st + 1 < nst) load(st + 1);
+        const double* const as = a0 + (st & 1) * 2 * TS * TFP;
+        const double* const bs = b0 + (st & 1) * 2 * TS * TFP;
+#pragma unroll
+        for (int kk = 0; kk < 16; kk += 8) {
+            double2_t av[2], bv[2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                av[t] = *(const double2_t*)(as + t * 16 * TFP + kk);
+                bv[t] = *(const double2_t*)(bs + t * 16 * TFP + kk);
+            }
+#pragma unroll
+            for (int a = 0; a < 2; a++)
+#pragma unroll
+                for (int c = 0; c < 2; c++) acc[a][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a].x, bv[c].x, acc[a][c], 0, 0, 0);
+#pragma unroll
+            for (int a = 0; a < 2; a++)
+#pragma unroll
+                for (int c = 0; c < 2; c++) acc[a][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a].y, bv[c].y, acc[a][c], 0, 0, 0);
+        }
+        if (st + 1 < nst) stage((st + 1) & 1);
+    }
+}
+// the accumulators of a tile at C (row pitch ldc): -C read, -acc written (its lower triangle only)
+__device__ __forceinline__ void load_neg(const double* C, size_t ldc, double4_t (&acc)[2][2])
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const double* const c0 = C + ((w >> 1) * 32 + (lane >> 4)) * ldc + (w & 1) * 32 + (lane & 15);
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) acc[a][c][v] = -c0[(a * 16 + 4 * v) * ldc + c * 16];
+}
+__device__ __forceinline__ void store_neg(double* C, size_t ldc, const double4_t (&acc)[2][2], bool lower)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int r0 = (w >> 1) * 32 + (lane >> 4), q0 = (w & 1) * 32 + (lane & 15);
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                if (!lower || q0 + c * 16 <= r0 + a * 16 + 4 * v) C[(r0 + a * 16 + 4 * v) * ldc + q0 + c * 16] = -acc[a][c][v];
+}
+// the diagonal block in sm's first 64 rows of DGP into the blocks of 16 columns, factored
+__device__ __forceinline__ void chol_diag_f64_lds(const MatDesc& D, int kb, double* tile, int ld, double* sm)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    __syncthreads();
+    double4_t acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) acc[i][v] = i >= w ? sm[(16 * i + 4 * v + (lane >> 4)) * DGP + 16 * w + (lane & 15)] : 0.0;
+    chol_diag_f64_4w(D, kb, tile, ld, acc, sm);
+}
+
+// Left-looking FP64 panel step: column block kb of the part that starts at k0, dense or banded (there
+// every earlier block of the row inside the band, so a banded factorization is one launch per column
+// block).  Workgroup y takes row block ib = kb + 1 + y and forms
+// L_ib,kb = (A_ib,kb - sum_k' L_ib,k' L_kb,k'^T) W_kb^T; the part's diagonal blocks (in a band, every
+// one of the launch) take this column's product at once, and the workgroup of ib = kb + 1 factors the
+// next one, so a column needs this one launch instead of a diagonal, a panel and a panel-update one.
+// Alone, a step is bound by that workgroup's serial chain (its 64^3 products at 1.7 us each on one CU,
+// then the diagonal block); the grid is (matrices, row blocks), so it is dispatched first.
+// One 3712 matrix alone: 4.3 -> 2.15 ms for the factorization, R's banded chain of 58 steps 3.0 -> 1.3.
+__global__ void __launch_bounds__(256) k_chol_lpanel_f64(const MatDesc* mats, int kb, int k0, int kend)
+{
+    __shared__ __attribute__((aligned(16))) double sm[DGL];  // stages, operand tiles, the diagonal block's buffers
+    static_assert(2 * 2 * 64 * TFP <= DGL && 2 * TS * LDT <= DGL, "the stages and the operand tiles fit");
+    double(*As)[LDT] = (double(*)[LDT])sm;
+    double(*Bs)[LDT] = (double(*)[LDT])(sm + TS * LDT);
+    const MatDesc D = mats[blockIdx.x];
+    if (kb >= D.nb) return;
+    const int ib = kb + 1 + blockIdx.y;
+    if (ib > band_last(D, kb)) return;
+    const int ks = D.bwb > 0 ? max(0, ib - D.bwb) : k0;
+    int ld, lp;
+    double* blk = tile_ptr<double>(D, ib, kb, ld);
+    double4_t acc[2][2];
+    load_neg(blk, ld, acc);
+    if (ks < kb) {
+        const long long bs = D.bwb > 0 ? -TS * TS : TS;
+        const double* Pa = tile_ptr<double>(D, ib, ks, lp);
+        gemm_f64(Pa, lp, bs, tile_ptr<double>(D, kb, ks, lp), lp, bs, 4 * (kb - ks), sm, acc);
+        __syncthreads();
+    }
+    stage64<double>((const double*)D.W + (size_t)kb * TS * TS, TS, Bs);
+    store_neg(&As[0][0], LDT, acc, false);
+    const bool upd = D.bwb > 0 || ib < kend;
+    double* dg = tile_ptr<double>(D, ib, ib, lp);
+    const int ldd = lp;
+    double4_t dacc[2][2];
+    if (upd) load_neg(dg, ldd, dacc);
+    __syncthreads();
+    mma64<double>(As, Bs, acc);  // L_ib,kb(i, j) = sum_q A'(i, q) W_kb(j, q)
+    store64<double>(blk, ld, acc);
+    if (!upd) return;
+    __syncthreads();
+    store64<double>(&As[0][0], LDT, acc);
+    __syncthreads();
+    mma64_add<double>(As, As, dacc);
+    if (ib != kb + 1) {
+        store_neg(dg, ldd, dacc, true);
+        return;
+    }
+    __syncthreads();
+    store_neg(sm, DGP, dacc, false);
+    chol_diag_f64_lds(D, ib, dg, ldd, sm);
+}
+
+// FP64 trailing update C(I, J) -= sum over the panel's nq column blocks of L(I, q) L(J, q)^T on the
+// 64-tiles of rows and columns >= k0 + nq; ncolt > 0: the first ncolt tile columns only, a strip.  The
+// accumulators start from -C and are stored negated, so each element takes its products in k order
+// whatever the panel's width.  Two LDS stages of 37 KB leave four workgroups a CU, so
+// that some multiply while others wait for their C tiles or store them: 52 TFLOP/s on 100 matrices of
+// 3712 (the 128-tile form with one workgroup of 139 KB a CU, whose C traffic stood beside the products:
+// 32; 128-tiles on the same two stages, two workgroups a CU: 50, and slower by 0.5 ms on one matrix).
+// fdiag (the diagonal block's buffers: two workgroups a CU) factors block k0 + nq in tile (0, 0)'s
+// workgroup; it saves the diagonal launch and its wait where the tiles do not fill those two anyway
+// (TRAIL_FUSED; 100 matrices of 3712: 38.5 ms fused, 34.9 apart; one: 2.15 against 2.23).
+#define TRAIL_F64_LDS (DGL * 8)
+#define TRAIL_F64_LDS0 (2 * 2 * 64 * TFP * 8)
+#define TRAIL_FUSED 512
+__global__ void __launch_bounds__(256) k_chol_trail_f64(const MatDesc* mats, int k0, int nq, int ncolt, int fdiag)
+{
+    extern __shared__ double trail_raw[];
+    const MatDesc D = mats[blockIdx.y];
+    const int r0b = k0 + nq;
+    if (r0b >= D.nb) return;
+    const int nt = D.nb - r0b;
+    int I = -1, J = -1;
+    if (ncolt == 0) {
+        if (!syrk_tile(nt, I, J)) return;
+    } else {
+        int t = blockIdx.x;
+        for (int j = 0; j < ncolt && j < nt; j++) {
+            if (t < nt - j) {
+                J = j;
+                I = j + t;
+                break;
+            }
+            t -= nt - j;
+        }
+        if (J < 0) return;
+    }
+    const size_t ld = D.ld;
+    double* const A = (double*)D.A;
+    const size_t rI = (size_t)(r0b + I) * TS, rJ = (size_t)(r0b + J) * TS;
+    double4_t acc[2][2];
+    load_neg(A + rI * ld + rJ, ld, acc);
+    gemm_f64(A + rI * ld + (size_t)k0 * TS, ld, TS, A + rJ * ld + (size_t)k0 * TS, ld, TS, 4 * nq, trail_raw, acc);
+    store_neg(A + rI * ld + rJ, ld, acc, I == J);
+    // fdiag: the workgroup of tile (0, 0) also factors diagonal block r0b, now up to date, so the part
+    // that starts there needs no diagonal launch
+    if (fdiag && I == 0 && J == 0) {
+        __syncthreads();
+        store_neg(trail_raw, DGP, acc, false);
+        chol_diag_f64_lds(D, r0b, A + rI * ld + rJ, (int)ld, trail_raw);
     }
 }
 
-// dense matrices (padded to a multiple of 128), factored panel by panel, each panel column block
-// by column block and then one trailing update of the rest.  FP32 (the mixed path, evaluated in
-// batches): 1024-wide panels of four 256-wide left-looking parts (the left-looking panel kernel
-// reads and writes each block once per column: 0.8 ms faster per batch of 64 3600 x 3600
-// matrices than the right-looking pair), each part after the first brought up to date by a strip
-// update from the earlier parts, then one rank-1024 BF16-split trailing update.  Per batch of 256
-// 3600 x 3600 matrices the factorization took 33.7 ms with a rank-256 update per 256 columns,
-// 30.0 ms with 512-wide panels and 29.4 ms with 1024-wide ones (2048: 29.1, one panel: 30.1; FP32
-// MFMA in the panel kernel then); the arithmetic, and so the result, is the same bit for bit.  FP64: 256-wide panels factored with the
-// right-looking panel and panel-update kernels, whose three times more workgroups fill the GPU
-// better when one matrix is factored alone (0.25 ms faster for one 3600 x 3600 matrix), and the
-// FP64 trailing update.  The schedule depends on the element type only, never on the batch, so an
-// item's arithmetic is the same alone and in any batch.
-#define QLX_CHOL_SUB 4  // 256-wide left-looking parts per FP32 panel
+// Dense matrices (padded to a multiple of 128), panel by panel of panel_blocks 64-blocks: each panel
+// in 256-wide left-looking parts, each part after the first brought up to date by a strip update from
+// the earlier parts, then one trailing update of the rest.  Only the first diagonal block has a launch
+// of its own: the others are factored by the panel step or the update before them.  FP32 (the mixed
+// path): per batch of 256 3600 x 3600 matrices the factorization took 33.7 ms with a rank-256 update
+// per 256 columns, 30.0 ms with 512-wide panels and 29.4 ms with 1024-wide ones (2048: 29.1, one panel:
+// 30.1; FP32 MFMA in the panel kernel then).  FP64: 1024-wide panels where there are many matrices (100
+// of 3712: 36.7 ms with 1024, 37.8 with 512, 40.1 with 256, which reads and writes the trailing matrix four
+// times as often), 256-wide ones for few (one of 3712: 2.15, 2.21 and 2.31 ms with 256, 512 and 1024: the
+// strips are launches on the serial chain); 60.9 and 4.3 ms with right-looking panels.  The schedule's
+// arithmetic does not depend on the panel's width or on the batch, so an item's factor is the same bits
+// alone and in any.
+#define CHOL_WIDE 16384  // matrices x blocks^2 from which FP64 panels are wide
+#define QLX_CHOL_SUB 4  // 256-wide left-looking parts per panel by default
 template <typename T>
 static void chol_two_level(hipStream_t s, const MatDesc* mats, int nmat, int max_nb, int panel_blocks)
 {
-    if (sizeof(T) == 4) {
-        const size_t lds_bf = (size_t)4 * TT * TBP * sizeof(uint16_t);
-        allow_big_lds((const void*)k_chol_trail_bf16);
-        const int NB = panel_blocks > 0 ? panel_blocks : 4 * QLX_CHOL_SUB;  // panel width in 64-blocks
-        for (int k0 = 0; k0 < max_nb; k0 += NB) {
-            for (int ks = k0; ks < k0 + NB && ks < max_nb; ks += 4) {
-                if (ks > k0) {  // the half's columns, from all earlier halves of the panel (a strip)
-                    const int nts = (max_nb - ks) / 2;
-                    hipLaunchKernelGGL(k_chol_trail_bf16, dim3(2 * nts - 1, nmat), dim3(256), lds_bf, s, mats, k0, ks - k0, 2, 1);
-                }
-                // the part's first diagonal block was factored by the strip or trailing update before it
-                chol_subpanel<T>(s, mats, nmat, max_nb, ks, ks + 4, true, ks > 0);
+    constexpr bool F32 = sizeof(T) == 4;
+    const size_t lds = (size_t)4 * TT * TBP * sizeof(uint16_t);
+    allow_big_lds(F32 ? (const void*)k_chol_trail_bf16 : (const void*)k_chol_trail_f64);
+    // the update of everything from block k0 + nq on, or (strip) of the first 256 columns there
+    auto trail = [&](int k0, int nq, bool strip) {
+        const int n = max_nb - k0 - nq, nt = n / 2;
+        if (F32) {
+            hipLaunchKernelGGL(k_chol_trail_bf16, dim3(strip ? 2 * nt - 1 : syrk_grid(nt), nmat), dim3(256), lds, s, mats, k0, nq, strip ? 2 : 0, 1);
+        } else {
+            const int grid = strip ? (n >= 4 ? 4 * n - 6 : n * (n + 1) / 2) : (int)syrk_grid(n);
+            const bool fused = (long long)(strip ? grid : n * (n + 1) / 2) * nmat <= TRAIL_FUSED;
+            hipLaunchKernelGGL(k_chol_trail_f64, dim3(grid, nmat), dim3(256), fused ? (size_t)TRAIL_F64_LDS : (size_t)TRAIL_F64_LDS0, s, mats,
+                               k0, nq, strip ? 4 : 0, fused ? 1 : 0);
+            if (!fused) hipLaunchKernelGGL(k_chol_diag4_m<T>, dim3(1, nmat), dim3(256), 0, s, mats, k0 + nq);
+        }
+    };
+    // panel width in 64-blocks
+    const int NB = panel_blocks > 0 ? panel_blocks : F32 || (long long)nmat * max_nb * max_nb >= CHOL_WIDE ? 4 * QLX_CHOL_SUB : 4;
+    hipLaunchKernelGGL(k_chol_diag4_m<T>, dim3(1, nmat), dim3(256), 0, s, mats, 0);
+    for (int k0 = 0; k0 < max_nb; k0 += NB) {
+        for (int ks = k0; ks < k0 + NB && ks < max_nb; ks += 4) {
+            if (ks > k0) trail(k0, ks - k0, true);  // the part's columns, from the panel's earlier parts
+            for (int kb = ks; kb < ks + 4 && kb + 1 < max_nb; kb++) {
+                const dim3 grid(nmat, max_nb - kb - 1);
+                if (F32) hipLaunchKernelGGL(k_chol_lpanel_bf16, grid, dim3(256), 0, s, mats, kb, ks, ks + 4);
+                else hipLaunchKernelGGL(k_chol_lpanel_f64, grid, dim3(256), 0, s, mats, kb, ks, ks + 4);
             }
-            if (k0 + NB >= max_nb) break;
-            const int nt = (max_nb - k0 - NB) / 2;
-            hipLaunchKernelGGL(k_chol_trail_bf16, dim3(syrk_grid(nt), nmat), dim3(256), lds_bf, s, mats, k0, NB, 0, 1);
         }
-        return;
-    }
-    const size_t lds = (size_t)2 * TT * LDT * sizeof(T);
-    allow_big_lds((const void*)k_chol_trail_m<T>);
-    for (int k0 = 0; k0 < max_nb; k0 += 4) {
-        chol_subpanel<T>(s, mats, nmat, max_nb, k0, k0 + 4, false);
-        if (k0 + 4 < max_nb) {
-            const int nt = (max_nb - k0 - 4) / 2;
-            hipLaunchKernelGGL(k_chol_trail_m<T>, dim3(syrk_grid(nt), nmat), dim3(256), lds, s, mats, k0, 4);
-        }
+        if (k0 + NB >= max_nb) break;
+        trail(k0, NB, false);
     }
 }
 
-// d_mats holds n32 FP32 matrices first, then n64 FP64 matrices.  Dense matrices (all of the
-// launch) use the two-level schedule; banded ones (lower band <= max_bwb blocks) the 64-block
-// right-looking one.
+// nmat matrices of one element type (f32): dense ones (all of the launch) by the two-level schedule,
+// banded ones (FP64, lower band <= max_bwb blocks) by one left-looking launch per column block
 void cholesky_batched(hipStream_t s, const MatDesc* d_mats, int n32, int n64, int max_nb, int dense, int max_bwb, int panel_blocks)
 {
     if (dense) {
@@ -2702,11 +2717,10 @@ void cholesky_batched(hipStream_t s, const MatDesc* d_mats, int n32, int n64, in
         if (n64) chol_two_level<double>(s, d_mats + n32, n64, max_nb, 0);
         return;
     }
-    for (int kb = 0; kb < max_nb; kb++) {
-        const int rest = std::min(max_nb - kb - 1, max_bwb);  // banded: at most max_bwb blocks below
-        if (n32) chol_step<float>(s, d_mats, n32, kb, rest);
-        if (n64) chol_step<double>(s, d_mats + n32, n64, kb, rest);
-    }
+    if (!n64) return;
+    hipLaunchKernelGGL(k_chol_diag4_m<double>, dim3(1, n64), dim3(256), 0, s, d_mats + n32, 0);
+    for (int kb = 0; kb + 1 < max_nb; kb++)
+        hipLaunchKernelGGL(k_chol_lpanel_f64, dim3(n64, std::min(max_nb - kb - 1, max_bwb)), dim3(256), 0, s, d_mats + n32, kb, 0, max_nb);
 }
 
 // 2 sum log(diag) in a fixed order (Cholesky_logdet_lower_packed, pixelgrid.cpp:17201-17210)

@@ -1,0 +1,48 @@
+"""FP64 factorizations at the sizes where their tiles, panels and bands end: F's blocked Cholesky
+(64-blocks padded to 128, 256-wide parts, narrow or wide panels) and R's banded one (bands from one to
+several blocks), against the oracle; and the same bits alone and in a batch large enough for the wide
+schedule."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from qlens_amd import qlx
+from qlens_amd import workloads as W
+
+# the oracle's factorization is the same arithmetic in another summation order: a few hundred roundings
+# of 1.1e-16 per entry, on systems of condition below 1e6
+TOL = 1e-9
+
+
+def _case(src_n):
+    case = W.c1()
+    case["src_n"] = src_n
+    return case
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("src_n", [(2, 2), (9, 7), (8, 8), (11, 11), (13, 10), (16, 16), (18, 14), (23, 22), (33, 31), (64, 6), (96, 8), (6, 64)])
+def test_factor_sizes_match_oracle(qlx_ctx, src_n):
+    case = _case(src_n)
+    data = O.mock_image(case)
+    ref, arr = O.invert(case, data)
+    qlx_ctx.load_workload(case, data)
+    r = qlx_ctx.invert_image_surface_brightness_map(case["lenses"])[0]
+    assert r["status"] == 0 and r["n_src_active"] == ref["n_src"]
+    for k in ("minus2lnE", "chisq0", "logdetF", "logdetR"):
+        assert abs(r[k] - ref[k]) <= TOL * max(1.0, abs(ref[k])), k
+    src = qlx_ctx.get_source()["src"]
+    assert np.linalg.norm(src - arr["src"]) <= TOL * np.linalg.norm(arr["src"])
+
+
+@pytest.mark.gpu
+def test_wide_panels_give_the_bits_of_narrow_ones(qlx_ctx):
+    case = _case((40, 36))  # 24 blocks: one matrix takes narrow panels, forty wide ones
+    data = O.mock_image(case)
+    qlx_ctx.load_workload(case, data)
+    models = W.proposals(case, 40, 5)
+    many = qlx_ctx.invert_image_surface_brightness_map(models)
+    for b in (0, 17, 39):
+        one = qlx_ctx.invert_image_surface_brightness_map(models[b])[0]
+        for k in ("minus2lnE", "logdetF", "logdetR", "Es"):
+            assert one[k] == many[b][k], (b, k)
