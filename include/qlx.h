@@ -341,11 +341,11 @@ int qlx_kernel_time(void *ctx, const char *name, double *ms, int *launches);
 
 /* Work counters of the last wave of the last qlx_eval (no reference counterpart; benchmark
  * accounting).  Sums over the wave's items unless noted:
- *   syrk_dense_flops   2*64^3 per (lower tile, 64-row chunk) pair of a dense SYRK
- *   syrk_exec_flops    MFMA flops executed: 2*64*CB^2 per pair of nonzero 64 x CB pool blocks
- *                      of one 64-row chunk (CB = 64 in FP64, 128 in MIXED; one product each)
+ *   syrk_dense_flops   2*64*16^2 per (lower pair of 16-column strips, 64-row chunk) of a dense SYRK
+ *   syrk_exec_flops    MFMA flops executed: the same per pair of 64 x 16 pool strips of one 64-row
+ *                      chunk (one product each)
  *   syrk_alg_flops     N_img*N_src*(N_src+1) + 2*N_img*N_src (the F and D arithmetic)
- *   lb_bytes           bytes of the blurred lensing matrix blocks written
+ *   lb_bytes           bytes of the blurred lensing matrix strips written
  *   integrand_evals    NFW integrand evaluations of the ray shooting
  *   chol_flops         N_src^3 / 3 (F's factorization; R's banded one is not counted)
  *   n_items            items of the wave

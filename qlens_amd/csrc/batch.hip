@@ -4,10 +4,10 @@
 // FP64 iterative refinement and the evidence terms.
 //
 // Item b of a batch is blockIdx.y (matrix index for the Cholesky kernels); per-item sizes and pool
-// offsets come from BatchDev::meta.  Layouts: Lb blocks are 64x64 row-major at
-// (chunk*ncb + colblock)*4096 of the item's pool; column n_src carries the data vector so the SYRK
-// also yields D = Lb^T C d (row n_src of F).  F and R are row-major ldN x ldN (lower triangle used),
-// padding beyond the source block is identity.
+// offsets come from BatchDev::meta.  Layouts: the blurred L is kept as strips of 64 rows (a chunk) x
+// 16 columns, only those a chunk's rows reach, a chunk's one after the other (k_build_lb_b); column n_src
+// carries the data vector so the SYRK also yields D = Lb^T C d (row n_src of F).  F is row-major
+// ldN x ldN (lower triangle used), R in banded 64 x 64 tiles, padding beyond the source block identity.
 //
 // Reference behaviour followed:
 //   active sets              assign_active_indices / assign_pixel_mappings  pixelgrid.cpp:3586-3626, 12879-12914
@@ -140,8 +140,8 @@ __global__ void __launch_bounds__(1024) k_compact_b(BatchDev bd)
     if (threadIdx.x == 0) bd.counts[4 * item] = base;
     __syncthreads();
     // internal order of F's source columns: the same active cells ranked tile by tile
-    // (QLX_TILE_W x QLX_TILE_H cells, tiles and cells inside a tile y-major), so that a compact
-    // source-plane patch occupies a compact index range
+    // (QLX_TILE_W x QLX_TILE_H cells; inside a tile 4 x 4 cells by 4 x 4 cells, all y-major), so that a
+    // compact source-plane patch occupies a compact index range, in strips of 16 as in blocks
     {
         int* tix = bd.tix + item * bd.s_cell;
         int* pis = bd.pisrc + item * bd.s_cell;
@@ -154,8 +154,9 @@ __global__ void __launch_bounds__(1024) k_compact_b(BatchDev bd)
             int c = -1, flag = 0;
             if (t < total) {
                 const int tile = t / tcells, wv = t - tile * tcells;
-                const int i = (tile % ntw) * QLX_TILE_W + wv % QLX_TILE_W;
-                const int j = (tile / ntw) * QLX_TILE_H + wv / QLX_TILE_W;
+                const int sub = wv >> 4;  // 4 x 4 cells each
+                const int i = (tile % ntw) * QLX_TILE_W + 4 * (sub % (QLX_TILE_W / 4)) + wv % 4;
+                const int j = (tile / ntw) * QLX_TILE_H + 4 * (sub / (QLX_TILE_W / 4)) + wv % 16 / 4;
                 if (i < snx && j < sny) {
                     c = i * sny + j;
                     flag = cm[c] ? 1 : 0;
@@ -274,16 +275,6 @@ __global__ void __launch_bounds__(256) k_merge_lrows_b(BatchDev bd)
                 }
             }
         }
-        unsigned m[QLX_MAX_CBW];
-#pragma unroll
-        for (int w = 0; w < QLX_MAX_CBW; w++) m[w] = 0;
-#pragma unroll
-        for (int j = 0; j < MU; j++)
-            if (j < n) {
-                const int cb = cols[j] >> M.cbs;
-#pragma unroll
-                for (int w = 0; w < QLX_MAX_CBW; w++) m[w] |= (w == (cb >> 5)) ? (1u << (cb & 31)) : 0u;
-            }
         if (nsub == 4) {  // the whole 12-slot row with vector stores (slots >= n: col -1, value 0, never read)
 #pragma unroll
             for (int j = 0; j < 3; j++) ((int4*)uc)[j] = make_int4(cols[4 * j], cols[4 * j + 1], cols[4 * j + 2], cols[4 * j + 3]);
@@ -298,10 +289,6 @@ __global__ void __launch_bounds__(256) k_merge_lrows_b(BatchDev bd)
                 }
         }
         bd.ucnt[item * bd.s_pix + r] = n;
-        unsigned* pm = bd.pmask + ((size_t)item * bd.s_pix + r) * QLX_MAX_CBW;
-#pragma unroll
-        for (int w = 0; w < QLX_MAX_CBW; w++)
-            if (w < M.ncbw) pm[w] = m[w];
         return;
     }
     int cnt = 0;
@@ -323,12 +310,6 @@ __global__ void __launch_bounds__(256) k_merge_lrows_b(BatchDev bd)
         }
     }
     bd.ucnt[item * bd.s_pix + r] = cnt;
-    unsigned* pm = bd.pmask + ((size_t)item * bd.s_pix + r) * QLX_MAX_CBW;
-    for (int w = 0; w < M.ncbw; w++) pm[w] = 0;
-    for (int e = 0; e < cnt; e++) {
-        const int cb = uc[e] >> M.cbs;
-        pm[cb >> 5] |= 1u << (cb & 31);
-    }
 }
 
 void launch_merge_lrows_b(hipStream_t s, const BatchDev& bd, int max_img)
@@ -576,110 +557,114 @@ void launch_lcols_b(hipStream_t s, const BatchDev& bd, int max_img, int max_src)
 }
 
 // ------------------------------------------------------------------------------------------------
-// chunk support: union of the 64-column blocks touched by the PSF taps of a chunk's 64 rows
-// (one workgroup per chunk), then per-item slot bases of the compact block pool.
+// chunk support (one workgroup per chunk): the columns of L with an entry in the PSF reach of the
+// chunk's 64 rows (a bit per column, which the Lb build also reads), the strips of 16 columns that
+// hold one (the pool holds these and only these), then per item the strips' slots and, per column
+// block of the SYRK, which strips of a chunk it holds and where they start.
 // ------------------------------------------------------------------------------------------------
-
-// m[o .. o+3] |= the four words of v.  Mask rows hold QLX_MAX_CBW = 8 words; words from ncbw on may
-// hold anything (they are never written to the support masks)
-static_assert(QLX_MAX_CBW == 8, "mask rows are read as two 16-byte vectors");
-__device__ __forceinline__ void or_mask4(unsigned (&m)[QLX_MAX_CBW], int o, uint4 v)
+__device__ __forceinline__ int wave_min_i(int v)
 {
-    m[o] |= v.x;
-    m[o + 1] |= v.y;
-    m[o + 2] |= v.z;
-    m[o + 3] |= v.w;
-}
-
-// PSF x window, per grid pixel t = y*nx + x: hmask[t] = OR of pmask over the active pixels x' in
-// [x + nxh - pnx + 1, x + nxh] of row y (one contiguous active-index range [apre[..i0], apre[..i1+1]))
-__global__ void __launch_bounds__(256) k_psf_hdilate_b(BatchDev bd)
-{
-    const int item = blockIdx.y;
-    const ItemMeta& M = bd.meta[item];
-    const int npix = bd.nx * bd.ny;
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (!M.valid || t >= npix) return;
-    const int y = t / bd.nx, x = t - y * bd.nx;
-    const int nxh = bd.pnx / 2;
-    const int i0 = max(0, x + nxh - bd.pnx + 1), i1 = min(bd.nx - 1, x + nxh);
-    const int* apre = bd.apre + item * (bd.s_pix + 1);
-    const unsigned* pm = bd.pmask + (size_t)item * bd.s_pix * QLX_MAX_CBW;
-    unsigned m[QLX_MAX_CBW];
 #pragma unroll
-    for (int w = 0; w < QLX_MAX_CBW; w++) m[w] = 0;
-    const int a0 = apre[y * bd.nx + i0], a1 = apre[y * bd.nx + i1 + 1];
-    const bool wide = M.ncbw > 4;  // mask rows are 32-byte aligned: one or two 16-byte loads per row
-    for (int a = a0; a < a1; a++) {
-        const uint4* p4 = (const uint4*)(pm + (size_t)a * QLX_MAX_CBW);
-        or_mask4(m, 0, p4[0]);
-        if (wide) or_mask4(m, 4, p4[1]);
-    }
-    uint4* h4 = (uint4*)(bd.hmask + ((size_t)item * bd.s_pix + t) * QLX_MAX_CBW);
-    h4[0] = make_uint4(m[0], m[1], m[2], m[3]);
-    if (wide) h4[1] = make_uint4(m[4], m[5], m[6], m[7]);
+    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
+    return v;
 }
-
-__global__ void __launch_bounds__(256) k_row_support_b(BatchDev bd)
+__device__ __forceinline__ int wave_max_i(int v)
 {
-    __shared__ unsigned msk[QLX_MAX_CBW];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+    return v;
+}
+// a chunk whose rows span at most LB_SPAN + 1 pixels each way is scanned as one rectangle, and the
+// padded tap table of the Lb build covers it
+#define LB_SPAN 15
+
+__global__ void __launch_bounds__(256) k_chunk_cols_b(BatchDev bd)
+{
+    extern __shared__ unsigned colbits[];  // M.ncw words
     __shared__ int rk[TS], rl[TS];
     const int item = blockIdx.y;
     const ItemMeta& M = bd.meta[item];
     const int kt = blockIdx.x;
     if (!M.valid || kt >= M.nkt) return;
-    const int tid = threadIdx.x;
-    if (tid < QLX_MAX_CBW) msk[tid] = 0;
+    const int tid = threadIdx.x, lane = tid & 63;
     const int rows = min(TS, M.n_img - kt * TS);
-    if (tid < rows) {
-        const int p = bd.act_pix[item * bd.s_pix + bd.perm[item * bd.s_pix + kt * TS + tid]];
-        rk[tid] = p / bd.ny;
-        rl[tid] = p - (p / bd.ny) * bd.ny;
+    for (int t = tid; t < M.ncw; t += 256) colbits[t] = 0u;
+    int k = 0, l = 0;
+    if (lane < rows) {
+        const int p = bd.act_pix[item * bd.s_pix + bd.perm[item * bd.s_pix + kt * TS + lane]];
+        k = p / bd.ny;
+        l = p - (p / bd.ny) * bd.ny;
+    }
+    if (tid < TS) {
+        rk[tid] = k;
+        rl[tid] = l;
+    }
+    const bool row = lane < rows;
+    const int kmin = wave_min_i(row ? k : 1 << 30), kmax = wave_max_i(row ? k : -(1 << 30));
+    const int lmin = wave_min_i(row ? l : 1 << 30), lmax = wave_max_i(row ? l : -(1 << 30));
+    __syncthreads();
+    const int U = 3 * bd.nsub, pnx = bd.pnx, pny = bd.pny;
+    const int* pidx = bd.pidx + item * bd.s_pix;
+    const int* ucnt = bd.ucnt + item * bd.s_pix;
+    const int* ucol = bd.ucol + (size_t)item * bd.s_pix * U;
+    auto mark = [&](int i, int j) {
+        if (i < 0 || i >= bd.nx || j < 0 || j >= bd.ny) return;
+        const int r = pidx[(size_t)i * bd.ny + j];
+        if (r < 0) return;
+        const int nu = ucnt[r];
+        for (int e = 0; e < nu; e++) {
+            const int c = ucol[(size_t)r * U + e];
+            atomicOr(&colbits[c >> 5], 1u << (c & 31));
+        }
+    };
+    // pixels (i, j) whose tap (k + hx - i, l + hy - j) lies in the PSF for a row (k, l): of a compact
+    // chunk the rectangle of all its rows' windows, otherwise row by row (a chunk of the last tiles of
+    // two image rows spans the image, not its pixels)
+    const int i0 = pnx / 2 - pnx + 1, j0 = pny / 2 - pny + 1;
+    if (kmax - kmin <= LB_SPAN && lmax - lmin <= LB_SPAN) {
+        const int wi = kmax - kmin + pnx, wj = lmax - lmin + pny;
+        for (int t = tid; t < wi * wj; t += 256) mark(kmin + i0 + t / wj, lmin + j0 + t % wj);
+    } else {
+        const int taps = pnx * pny;
+        for (int t = tid; t < rows * taps; t += 256) {
+            const int rr = t / taps, q = t - rr * taps;
+            mark(rk[rr] + i0 + q / pny, rl[rr] + j0 + q % pny);
+        }
     }
     __syncthreads();
-    unsigned m[QLX_MAX_CBW];
-#pragma unroll
-    for (int w = 0; w < QLX_MAX_CBW; w++) m[w] = 0;
-    {
-        const int cbd = M.n_src >> M.cbs;  // the data column (thread 0)
-#pragma unroll
-        for (int w = 0; w < QLX_MAX_CBW; w++) m[w] |= (tid == 0 && w == (cbd >> 5)) ? (1u << (cbd & 31)) : 0u;
+    unsigned* cb = bd.colb + M.col_off + (size_t)kt * M.ncw;
+    for (int t = tid; t < M.ncw; t += 256) cb[t] = colbits[t];
+    // strip s = columns 16 s .. 16 s + 15; the data column's strip is in every chunk
+    if (tid < M.nsw) {
+        unsigned m = 0;
+        for (int q = 0; q < 16 && 16 * tid + q < M.ncw; q++) {
+            const unsigned c = colbits[16 * tid + q];
+            m |= ((c & 0xffffu) ? 1u : 0u) << (2 * q) | ((c >> 16) ? 1u : 0u) << (2 * q + 1);
+        }
+        const int sd = M.n_src >> 4;
+        if ((sd >> 5) == tid) m |= 1u << (sd & 31);
+        bd.nz[M.nz_off + (size_t)kt * M.nsw + tid] = m;
     }
-    const int nyh = bd.pny / 2;
-    const unsigned* hm = bd.hmask + (size_t)item * bd.s_pix * QLX_MAX_CBW;
-    // (row, window row) pairs: the PSF window of row (k, l) at y = l + nyh - pl is the x-window
-    // union already held by hmask[y*nx + k]
-    for (int q = tid; q < rows * bd.pny; q += 256) {
-        const int rr = q / bd.pny, pl = q - rr * bd.pny;
-        const int jj = rl[rr] + nyh - pl;
-        if (jj < 0 || jj >= bd.ny) continue;
-        const uint4* h4 = (const uint4*)(hm + ((size_t)jj * bd.nx + rk[rr]) * QLX_MAX_CBW);
-        or_mask4(m, 0, h4[0]);
-        if (M.ncbw > 4) or_mask4(m, 4, h4[1]);
-    }
-#pragma unroll
-    for (int w = 0; w < QLX_MAX_CBW; w++)
-        if (m[w]) atomicOr(&msk[w], m[w]);
-    __syncthreads();
-    if (tid < M.ncbw) bd.nz[M.nz_off + (size_t)kt * M.ncbw + tid] = msk[tid];
 }
 
+// the chunks' first slots in the item's pool (in strips), the item's strips and its strip pairs
 __global__ void __launch_bounds__(1024) k_block_scan_b(BatchDev bd)
 {
     __shared__ int sh[40];
-    __shared__ int smax[1024];
+    __shared__ unsigned long long sp[1024];
     const int item = blockIdx.y;
     const ItemMeta& M = bd.meta[item];
     if (!M.valid) return;
     const unsigned* nz = bd.nz + M.nz_off;
     int* bb = bd.bbase + M.bb_off;
-    int base = 0, best = 0;
+    int base = 0;
+    unsigned long long pairs = 0;
     for (int t0 = 0; t0 < M.nkt; t0 += 1024) {
         const int t = t0 + threadIdx.x;
         int v = 0;
         if (t < M.nkt)
-            for (int w = 0; w < M.ncbw; w++) v += __popc(nz[(size_t)t * M.ncbw + w]);
-        best = max(best, v);
+            for (int w = 0; w < M.nsw; w++) v += __popc(nz[(size_t)t * M.nsw + w]);
+        pairs += (unsigned long long)v * (v + 1) / 2;
         const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
         int incl = wave_incl_scan(v);
         if (lane == 63) sh[wv] = incl;
@@ -696,53 +681,65 @@ __global__ void __launch_bounds__(1024) k_block_scan_b(BatchDev bd)
         __syncthreads();
         base += tot;
     }
-    smax[threadIdx.x] = best;
+    sp[threadIdx.x] = pairs;
     __syncthreads();
     for (int st = 512; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st) smax[threadIdx.x] = max(smax[threadIdx.x], smax[threadIdx.x + st]);
+        if ((int)threadIdx.x < st) sp[threadIdx.x] += sp[threadIdx.x + st];
         __syncthreads();
     }
     if (threadIdx.x == 0) {
         bb[M.nkt] = base;
         bd.counts[4 * item + 2] = base;
-        bd.counts[4 * item + 3] = smax[0];
+        bd.npairs[item] = sp[0];
     }
 }
 
-void launch_row_support_b(hipStream_t s, const BatchDev& bd, int max_nkt)
+// sup[I * nkt + kt]: of chunk kt's strips those in column block I (1 << cbs columns): mask in the low
+// byte, their first strip's rank in the chunk above it; 0 where there is none
+__global__ void __launch_bounds__(256) k_sup_table_b(BatchDev bd)
+{
+    const int item = blockIdx.y;
+    const ItemMeta& M = bd.meta[item];
+    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (!M.valid || t >= (long long)M.ncb * M.nkt) return;
+    const int I = (int)(t / M.nkt), kt = (int)(t - (long long)I * M.nkt);
+    const unsigned* m = bd.nz + M.nz_off + (size_t)kt * M.nsw;
+    const int sb = 1 << (M.cbs - 4), s0 = I * sb;  // 4 or 8 strips a block: within one word
+    unsigned rank = 0;
+    for (int w = 0; w < (s0 >> 5); w++) rank += __popc(m[w]);
+    const unsigned word = m[s0 >> 5];
+    rank += __popc(word & ((1u << (s0 & 31)) - 1u));
+    const unsigned mask = (word >> (s0 & 31)) & ((1u << sb) - 1u);
+    bd.sup[M.sup_off + t] = mask ? rank << 8 | mask : 0u;
+}
+
+void launch_row_support_b(hipStream_t s, const BatchDev& bd, int max_nkt, int max_ld, int max_sup)
 {
     if (max_nkt <= 0) return;
-    const int npix = bd.nx * bd.ny;
-    hipLaunchKernelGGL(k_psf_hdilate_b, dim3((npix + 255) / 256, bd.B), dim3(256), 0, s, bd);
-    hipLaunchKernelGGL(k_row_support_b, dim3(max_nkt, bd.B), dim3(256), 0, s, bd);
+    hipLaunchKernelGGL(k_chunk_cols_b, dim3(max_nkt, bd.B), dim3(256), (size_t)max_ld / 8, s, bd);
     hipLaunchKernelGGL(k_block_scan_b, dim3(1, bd.B), dim3(1024), 0, s, bd);
+    hipLaunchKernelGGL(k_sup_table_b, dim3((max_sup + 255) / 256, bd.B), dim3(256), 0, s, bd);
 }
-
-// rank of block cb among the set bits of a chunk's support mask
-__device__ __forceinline__ int mask_rank(const unsigned* m, int cb)
-{
-    int s = 0;
-    for (int w = 0; w < (cb >> 5); w++) s += __popc(m[w]);
-    return s + __popc(m[cb >> 5] & ((1u << (cb & 31)) - 1u));
-}
-__device__ __forceinline__ bool mask_has(const unsigned* m, int cb) { return (m[cb >> 5] >> (cb & 31)) & 1u; }
 
 // ------------------------------------------------------------------------------------------------
-// Blurred rows of one 64-row chunk into the chunk's support blocks (PSF_convolution_Lmatrix_dense,
+// Blurred rows of one 64-row chunk into the chunk's support strips (PSF_convolution_Lmatrix_dense,
 // direct branch, pixelgrid.cpp:14092-14176): Lb[r][c] = sum over pixels (i, j) of the chunk's PSF
 // reach of psf[k_r + hx - i][l_r + hy - j] * L[(i, j)][c], taps inside the PSF only, (i, j) active.
 // One workgroup per chunk; lane l of every wave owns chunk row l (the rows are image-compact, so an
-// L entry of a pixel near the chunk reaches most of its rows).  Per support column c (columns of a
-// block dealt to the four waves), the wave walks column c's entries in L's CSC form, keeps those
-// whose pixel lies in the chunk's PSF reach (a ballot over 64 entries at a time), broadcasts each
-// kept entry and every lane adds its own tap weight times the value: the output element is summed
-// in registers in a fixed order and written once, with no atomics.  A block's 64 x CB values go to
-// an LDS tile and from there to the pool with 16-byte stores.
-//   T = double: FP64 pool, 64-column blocks, row-major, unscaled (the FP64 SYRK applies C);
-//   T = float:  FP16 pool, 128-column blocks, k4-interleaved (element (k, i) at
-//               ((k >> 2) * CB + i) * 4 + (k & 3), so the SYRK stages blocks with 16-byte copies),
-//               entries x = Lb sqrt(c_r) s16 rounded once (s16 a power of two, |x| <= 2^14).
-// Column n_src carries the data: d (FP64) or d sqrt(c_r) s16 (FP16).
+// L entry of a pixel near the chunk reaches most of its rows), and a wave takes every fourth of the
+// chunk's strips of 16 columns.  Per column with an entry in the reach (colb) it walks the column's
+// entries in L's CSC form, keeps those whose pixel lies in the reach (a ballot over 64 entries at a
+// time), broadcasts each kept entry and every lane adds its own tap weight times the value: the output
+// element is summed in registers in a fixed order and written once, with no atomics.  A strip's values
+// go to the wave's LDS tile and from there to the pool with 16-byte stores; waves share no barrier.
+//   T = double: FP64 pool, unscaled (the FP64 SYRK applies C), a strip's element (row k, column i) at
+//               ((k >> 1) * 16 + i) * 2 + (k & 1): a lane's 16 bytes are two rows of its column;
+//   T = float:  FP16 pool, ((k >> 3) * 16 + i) * 8 + (k & 7): a lane's 16 bytes are the eight rows of
+//               an MFMA operand; entries x = Lb sqrt(c_r) s16 rounded once (s16 a power of two, |x| <=
+//               2^14).
+// Column n_src carries the data: d (FP64) or d sqrt(c_r) s16 (FP16).  256 items of the 200 x 200 / 60 x 60
+// workload: 9.8 ms with half blocks of 64 columns shared by the four waves and stored whole (12.8 GB),
+// 6.7 on strips (5.6 GB), both FP16; bound by its LDS traffic (a broadcast and 64 tap reads per kept entry).
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ uint16_t f32_to_f16_rne(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
 
@@ -761,19 +758,6 @@ template <typename T> __device__ __forceinline__ T readlane_t(T v, int l);
 template <> __device__ __forceinline__ double readlane_t<double>(double v, int l) { return readlane_f64(v, l); }
 template <> __device__ __forceinline__ float readlane_t<float>(float v, int l) { return readlane_f32(v, l); }
 
-__device__ __forceinline__ int wave_min_i(int v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
-    return v;
-}
-__device__ __forceinline__ int wave_max_i(int v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
 // Tap table in LDS: tap (tp, tq) of the PSF at (tp + toff) * tpc + tq.  Padded form (toff =
 // LB_SPAN + 1, tpc >= pny + LB_SPAN + 1, pnx + 2 LB_SPAN + 2 rows, zero outside the PSF): for a chunk
 // whose rows span at most LB_SPAN + 1 pixels in each direction, every kept L entry (i, j) of the
@@ -784,7 +768,6 @@ __device__ __forceinline__ int wave_max_i(int v)
 // before): no bounds test, and the zero products add exact zeros, so the sums are the bounds-tested
 // ones bit for bit.  Other chunks (and PSFs too large for the padded table: compact form, toff = 0,
 // tpc = pny) test the bounds per entry.
-#define LB_SPAN 15
 
 template <typename T>
 struct LbEnt {
@@ -799,158 +782,32 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Half h (CB/2 columns) of support block cb of a chunk by columns: wave w takes the half's columns
-// w + 4 l; lane = chunk row.  Per column the wave walks the column's entries in L's CSC form, keeps
-// those whose pixel lies in the chunk's PSF reach (a ballot over 64 entries at a time) and every lane
-// adds its own tap weight times each kept value, in the entries' order.  Fast chunks pass the kept
-// entries (E, value) through the wave's LDS slots (ent) and read the padded table at K - E; the
-// others broadcast each entry by readlane and test the tap's bounds.  Writes the half block's image
-// into `tile` (no barrier inside).
+// LDS tile of a wave: eight columns of a strip as runs of eight 16-byte pieces (one per FP64 row pair or
+// FP16 group of eight rows), 16 bytes of padding a run: at a multiple of 128 bytes the lanes' stores of a
+// column fell on the same banks
 template <typename T>
-__device__ __forceinline__ void lb_half(const BatchDev& bd, const ItemMeta& M, const T* tab, int toff, int tpc, LbEnt<T>* ent,
-                                        const unsigned* colbits, char* tile, int cb, int h, int w, int lane, int p, int kr2,
-                                        int lr2, int K, bool fast, int i_lo, unsigned i_span, int j_lo, unsigned j_span,
-                                        double sc, double dv, const unsigned* cpix, const double* cval, const int* cptr)
-{
-    constexpr bool F64 = sizeof(T) == 8;
-    const int cbs = M.cbs, CB = 1 << cbs, HB = CB >> 1;
-    const int pnx = bd.pnx, pny = bd.pny;
-    const int ncol = HB / 4;
-    const int c0h = (cb << cbs) + h * HB;
-    const int cl = c0h + w + 4 * lane;
-    int lb0 = 0, lb1 = 0;
-    if (lane < ncol && cl < M.n_src) {
-        lb0 = cptr[cl];
-        lb1 = cptr[cl + 1];
-    }
-    // the wave's columns with an entry in the chunk's reach (and the data column n_src): the others
-    // sum nothing, and their outputs are written directly
-    const bool live = lane < ncol && (cl == M.n_src || (cl < M.n_src && ((colbits[cl >> 5] >> (cl & 31)) & 1u)));
-    unsigned long long lmask = __ballot(live);
-    int nxt = lmask ? __builtin_ctzll(lmask) : ncol;
-    int ce0 = 0, ce1 = 0;
-    unsigned pk = 0;
-    double vd = 0.0;
-    if (nxt < ncol) {
-        ce0 = __builtin_amdgcn_readlane(lb0, nxt);
-        ce1 = __builtin_amdgcn_readlane(lb1, nxt);
-        if (ce0 + lane < ce1) {
-            pk = cpix[ce0 + lane];
-            vd = cval[ce0 + lane];
-        }
-    }
-    for (int l = 0; l < ncol; l++) {
-        const int ii = w + 4 * l;
-        if (l != nxt) {  // no entry in reach: acc = 0
-            const int c_ = c0h + ii;
-            if constexpr (F64) {
-                ((double*)tile)[lane * (HB + 2) + ii] = c_ == M.n_src ? dv : 0.0;
-            } else {
-                const double x = c_ == M.n_src ? dv : 0.0 * sc;
-                ((uint16_t*)tile)[((lane >> 2) * (HB + 2) + ii) * 4 + (lane & 3)] = f32_to_f16_rne((float)x);
-            }
-            continue;
-        }
-        lmask &= lmask - 1;
-        nxt = lmask ? __builtin_ctzll(lmask) : ncol;
-        const int e0c = ce0, e1c = ce1;
-        unsigned pkc = pk;
-        double vc = vd;
-        pk = 0;
-        vd = 0.0;
-        if (nxt < ncol) {
-            ce0 = __builtin_amdgcn_readlane(lb0, nxt);
-            ce1 = __builtin_amdgcn_readlane(lb1, nxt);
-            if (ce0 + lane < ce1) {
-                pk = cpix[ce0 + lane];
-                vd = cval[ce0 + lane];
-            }
-        }
-        T acc = (T)0;
-        for (int e0 = e0c; e0 < e1c; e0 += 64) {
-            if (e0 != e0c) {
-                pkc = 0;
-                vc = 0.0;
-                if (e0 + lane < e1c) {
-                    pkc = cpix[e0 + lane];
-                    vc = cval[e0 + lane];
-                }
-            }
-            const bool rel = e0 + lane < e1c && (unsigned)((int)(pkc >> 16) - i_lo) <= i_span &&
-                             (unsigned)((int)(pkc & 0xffffu) - j_lo) <= j_span;
-            const T v = (T)vc;
-            unsigned long long bal = __ballot(rel);
-            if (fast) {
-                if (rel) {
-                    const int pos = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
-                    ent[pos].e = ((int)(pkc >> 16) * tpc + (int)(pkc & 0xffffu)) * (int)sizeof(T);
-                    ent[pos].v = v;
-                }
-                wave_lds_sync();
-                const int n = __popcll(bal);
-                const char* tb = (const char*)tab + K * (int)sizeof(T);  // byte offsets: tap at tb - E
-                int k = 0;
-                if constexpr (sizeof(T) == 4) {
-                    // two entries per 16-byte LDS read (the same value in every lane)
-                    for (; k + 4 <= n; k += 4) {
-                        const uint4 q0 = *(const uint4*)&ent[k], q1 = *(const uint4*)&ent[k + 2];
-                        const T t0 = *(const T*)(tb - (int)q0.x), t1 = *(const T*)(tb - (int)q0.z);
-                        const T t2 = *(const T*)(tb - (int)q1.x), t3 = *(const T*)(tb - (int)q1.z);
-                        acc += t0 * __uint_as_float(q0.y);
-                        acc += t1 * __uint_as_float(q0.w);
-                        acc += t2 * __uint_as_float(q1.y);
-                        acc += t3 * __uint_as_float(q1.w);
-                    }
-                }
-                for (; k + 4 <= n; k += 4) {  // four entries' reads in flight together, summed in order
-                    const LbEnt<T> x0 = ent[k], x1 = ent[k + 1], x2 = ent[k + 2], x3 = ent[k + 3];
-                    const T t0 = *(const T*)(tb - x0.e), t1 = *(const T*)(tb - x1.e);
-                    const T t2 = *(const T*)(tb - x2.e), t3 = *(const T*)(tb - x3.e);
-                    acc += t0 * x0.v;
-                    acc += t1 * x1.v;
-                    acc += t2 * x2.v;
-                    acc += t3 * x3.v;
-                }
-                for (; k < n; k++) acc += *(const T*)(tb - ent[k].e) * ent[k].v;
-                wave_lds_sync();
-            } else {
-                while (bal) {
-                    const int b = __builtin_ctzll(bal);
-                    bal &= bal - 1;
-                    const unsigned pkb = (unsigned)__builtin_amdgcn_readlane((int)pkc, b);
-                    const T vb = readlane_t<T>(v, b);
-                    const int tp = kr2 - (int)(pkb >> 16), tq = lr2 - (int)(pkb & 0xffffu);
-                    if (p >= 0 && (unsigned)tp < (unsigned)pnx && (unsigned)tq < (unsigned)pny) acc += tab[(tp + toff) * tpc + tq] * vb;
-                }
-            }
-        }
-        if (p < 0) acc = (T)0;  // rows past the image: the fast path read row 0's taps for them
-        const int c_ = c0h + ii;
-        if constexpr (F64) {
-            ((double*)tile)[lane * (HB + 2) + ii] = c_ == M.n_src ? dv : (double)acc;
-        } else {
-            const double x = c_ == M.n_src ? dv : (double)acc * sc;
-            ((uint16_t*)tile)[((lane >> 2) * (HB + 2) + ii) * 4 + (lane & 3)] = f32_to_f16_rne((float)x);
-        }
-    }
-}
+struct LbTile {
+    static constexpr int RPR = 16 / (sizeof(T) == 8 ? 8 : 2);  // rows per run
+    static constexpr int NRUN = TS / RPR;
+    static constexpr int HC = 8;                               // columns per tile
+    static constexpr int PITCH = 128 + 16;                     // bytes
+    static constexpr int BYTES = NRUN * PITCH;
+};
 
 template <typename T>
-__global__ void __launch_bounds__(256) k_build_lb_b(BatchDev bd, int tab_bytes, int toff, int tpc, int trows, int nbw)
+__global__ void __launch_bounds__(256) k_build_lb_b(BatchDev bd, int tab_bytes, int toff, int tpc, int trows)
 {
     extern __shared__ double lds_raw[];
     const int item = blockIdx.y, kt = blockIdx.x;
     const ItemMeta& M = bd.meta[item];
     if (!M.valid || kt >= M.nkt) return;
     constexpr bool F64 = sizeof(T) == 8;
-    const int cbs = M.cbs, CB = 1 << cbs, HB = CB >> 1;
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    typedef LbTile<T> LT;
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int pnx = bd.pnx, pny = bd.pny;
     T* tab = (T*)lds_raw;
-    LbEnt<T>* ents = (LbEnt<T>*)((char*)lds_raw + tab_bytes);
-    unsigned* colbits = (unsigned*)(ents + 4 * 64);  // nbw words: columns with an entry in the reach
-    char* tile = (char*)(colbits + nbw);
-    for (int t = tid; t < nbw; t += 256) colbits[t] = 0u;
+    LbEnt<T>* ent = (LbEnt<T>*)((char*)lds_raw + tab_bytes) + 64 * w;
+    char* tile = (char*)lds_raw + tab_bytes + 4 * 64 * sizeof(LbEnt<T>) + w * LT::BYTES;
     for (int t = tid; t < trows * tpc; t += 256) {
         const int tr = t / tpc, tq = t - tr * tpc, tp = tr - toff;
         tab[t] = (tp >= 0 && tp < pnx && tq < pny) ? (T)bd.psf[tp * pny + tq] : (T)0;
@@ -978,67 +835,146 @@ __global__ void __launch_bounds__(256) k_build_lb_b(BatchDev bd, int tab_bytes, 
             dv = bd.data[p] * sc;
         }
     }
-    const unsigned* m = bd.nz + M.nz_off + (size_t)kt * M.ncbw;
-    const int sbase = bd.bbase[M.bb_off + kt];
-    const size_t bsz = (size_t)TS * CB;  // elements of one pool block
+    const unsigned* m = bd.nz + M.nz_off + (size_t)kt * M.nsw;
+    const unsigned* cb = bd.colb + M.col_off + (size_t)kt * M.ncw;
     const size_t eb = (size_t)item * bd.s_pix * 3 * bd.nsub;
     const unsigned* cpix = bd.cpix + eb;
     const double* cval = bd.cval + eb;
     const int* cptr = bd.boff + item * (bd.s_cell + 2);
-    LbEnt<T>* ent = ents + 64 * w;
-    __syncthreads();  // colbits cleared
-    // the columns of the L rows of the active pixels in the chunk's reach (the rectangle the CSC
-    // filter below keeps): exactly the columns with at least one kept entry
-    {
-        const int U = 3 * bd.nsub, wj = (int)j_span + 1;
-        const int nrect = ((int)i_span + 1) * wj;
-        const int* pidx = bd.pidx + item * bd.s_pix;
-        const int* ucnt = bd.ucnt + item * bd.s_pix;
-        const int* ucol = bd.ucol + (size_t)item * bd.s_pix * U;
-        for (int t = tid; t < nrect; t += 256) {
-            const int i = i_lo + t / wj, j = j_lo + t % wj;
-            if (i < 0 || i >= bd.nx || j < 0 || j >= bd.ny) continue;
-            const int r = pidx[(size_t)i * bd.ny + j];
-            if (r < 0) continue;
-            const int nu = ucnt[r];
-            for (int e = 0; e < nu; e++) {
-                const int c = ucol[(size_t)r * U + e];
-                atomicOr(&colbits[c >> 5], 1u << (c & 31));
-            }
-        }
-    }
-    __syncthreads();
-    // a half block's image: runs of HB * 8 bytes (FP64: 64 rows; FP16: 16 groups of 4 rows, the
-    // k4-interleaved layout), each landing at byte 8 (run * CB + h * HB) of the pool block.  In LDS
-    // the runs are HB * 8 + 16 bytes apart: at HB * 8 bytes (a multiple of 256) every lane's store of
-    // a column fell on the same two banks
-    const int nrun = F64 ? TS : TS / 4, upr = HB / 2;
+    // a strip's 64 x 16 elements are 128 16-byte pieces (FP16) or 512 (FP64)
+    uint4* dst0 = (uint4*)((char*)bd.lb + M.lb_off * (F64 ? 8 : 2)) + (size_t)bd.bbase[M.bb_off + kt] * (F64 ? 512 : 128);
+    const char* const tb = (const char*)tab + K * (int)sizeof(T);  // byte offsets: tap at tb - E
+    __syncthreads();  // the table
     int q = 0;
-    for (int wd = 0; wd < M.ncbw; wd++) {
+    for (int wd = 0; wd < M.nsw; wd++) {
         unsigned bits = m[wd];
         while (bits) {
-            const int cb = wd * 32 + __builtin_ctz(bits);
+            const int strip = wd * 32 + __builtin_ctz(bits);
             bits &= bits - 1;
-            uint4* dst = (uint4*)((char*)bd.lb + (M.lb_off + (size_t)(sbase + q) * bsz) * (F64 ? 8 : 2));
-            for (int h = 0; h < 2; h++) {
-                lb_half<T>(bd, M, tab, toff, tpc, ent, colbits, tile, cb, h, w, lane, p, kr2, lr2, K, fast, i_lo, i_span,
-                           j_lo, j_span, sc, dv, cpix, cval, cptr);
-                __syncthreads();
-                const uint4* src = (const uint4*)tile;
-                for (int u = tid; u < nrun * upr; u += 256) {
-                    const int run = u >> (cbs - 2), o = u & (upr - 1);  // upr = 2^(cbs - 2)
-                    store_nt(&dst[(run * CB + h * HB) / 2 + o], src[run * (upr + 1) + o]);
-                }
-                __syncthreads();
+            if ((q++ & 3) != w) continue;
+            const int c0 = 16 * strip;
+            const unsigned live16 = (cb[strip >> 1] >> (16 * (strip & 1))) & 0xffffu;
+            int lb0 = 0, lb1 = 0;
+            if (lane < 16 && c0 + lane < M.n_src) {
+                lb0 = cptr[c0 + lane];
+                lb1 = cptr[c0 + lane + 1];
             }
-            q++;
+#pragma unroll 1
+            for (int h = 0; h < 16; h += LT::HC) {
+                unsigned lmask = (live16 >> h) & ((1u << LT::HC) - 1u);
+                int nxt = lmask ? __builtin_ctz(lmask) : LT::HC;
+                int ce0 = 0, ce1 = 0;
+                unsigned pk = 0;
+                double vd = 0.0;
+                if (nxt < LT::HC) {
+                    ce0 = __builtin_amdgcn_readlane(lb0, h + nxt);
+                    ce1 = __builtin_amdgcn_readlane(lb1, h + nxt);
+                    if (ce0 + lane < ce1) {
+                        pk = cpix[ce0 + lane];
+                        vd = cval[ce0 + lane];
+                    }
+                }
+                // columns without an entry in the reach are zero
+                for (int t = lane; t < LT::NRUN * 8; t += 64) *(uint4*)(tile + (t >> 3) * LT::PITCH + (t & 7) * 16) = make_uint4(0, 0, 0, 0);
+                wave_lds_sync();
+                while (nxt < LT::HC) {
+                    const int ii = nxt;
+                    lmask &= lmask - 1;
+                    nxt = lmask ? __builtin_ctz(lmask) : LT::HC;
+                    const int e0c = ce0, e1c = ce1;
+                    unsigned pkc = pk;
+                    double vc = vd;
+                    pk = 0;
+                    vd = 0.0;
+                    if (nxt < LT::HC) {  // the next live column's first entries
+                        ce0 = __builtin_amdgcn_readlane(lb0, h + nxt);
+                        ce1 = __builtin_amdgcn_readlane(lb1, h + nxt);
+                        if (ce0 + lane < ce1) {
+                            pk = cpix[ce0 + lane];
+                            vd = cval[ce0 + lane];
+                        }
+                    }
+                    T acc = (T)0;
+                    for (int e0 = e0c; e0 < e1c; e0 += 64) {
+                        if (e0 != e0c) {
+                            pkc = 0;
+                            vc = 0.0;
+                            if (e0 + lane < e1c) {
+                                pkc = cpix[e0 + lane];
+                                vc = cval[e0 + lane];
+                            }
+                        }
+                        const bool rel = e0 + lane < e1c && (unsigned)((int)(pkc >> 16) - i_lo) <= i_span &&
+                                         (unsigned)((int)(pkc & 0xffffu) - j_lo) <= j_span;
+                        const T v = (T)vc;
+                        unsigned long long bal = __ballot(rel);
+                        if (fast) {
+                            if (rel) {
+                                const int pos = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
+                                ent[pos].e = ((int)(pkc >> 16) * tpc + (int)(pkc & 0xffffu)) * (int)sizeof(T);
+                                ent[pos].v = v;
+                            }
+                            wave_lds_sync();
+                            const int n = __popcll(bal);
+                            int k = 0;
+                            if constexpr (sizeof(T) == 4) {
+                                // two entries per 16-byte LDS read (the same value in every lane)
+                                for (; k + 4 <= n; k += 4) {
+                                    const uint4 q0 = *(const uint4*)&ent[k], q1 = *(const uint4*)&ent[k + 2];
+                                    const T t0 = *(const T*)(tb - (int)q0.x), t1 = *(const T*)(tb - (int)q0.z);
+                                    const T t2 = *(const T*)(tb - (int)q1.x), t3 = *(const T*)(tb - (int)q1.z);
+                                    acc += t0 * __uint_as_float(q0.y);
+                                    acc += t1 * __uint_as_float(q0.w);
+                                    acc += t2 * __uint_as_float(q1.y);
+                                    acc += t3 * __uint_as_float(q1.w);
+                                }
+                            }
+                            for (; k + 4 <= n; k += 4) {  // four entries' reads in flight together, summed in order
+                                const LbEnt<T> x0 = ent[k], x1 = ent[k + 1], x2 = ent[k + 2], x3 = ent[k + 3];
+                                const T t0 = *(const T*)(tb - x0.e), t1 = *(const T*)(tb - x1.e);
+                                const T t2 = *(const T*)(tb - x2.e), t3 = *(const T*)(tb - x3.e);
+                                acc += t0 * x0.v;
+                                acc += t1 * x1.v;
+                                acc += t2 * x2.v;
+                                acc += t3 * x3.v;
+                            }
+                            for (; k < n; k++) acc += *(const T*)(tb - ent[k].e) * ent[k].v;
+                            wave_lds_sync();
+                        } else {
+                            while (bal) {
+                                const int b = __builtin_ctzll(bal);
+                                bal &= bal - 1;
+                                const unsigned pkb = (unsigned)__builtin_amdgcn_readlane((int)pkc, b);
+                                const T vb = readlane_t<T>(v, b);
+                                const int tp = kr2 - (int)(pkb >> 16), tq = lr2 - (int)(pkb & 0xffffu);
+                                if (p >= 0 && (unsigned)tp < (unsigned)pnx && (unsigned)tq < (unsigned)pny) acc += tab[(tp + toff) * tpc + tq] * vb;
+                            }
+                        }
+                    }
+                    if (p < 0) acc = (T)0;  // rows past the image: the fast path read row 0's taps for them
+                    char* d = tile + lane / LT::RPR * LT::PITCH + ii * 16 + lane % LT::RPR * (16 / LT::RPR);
+                    if constexpr (F64) *(double*)d = acc;
+                    else *(uint16_t*)d = f32_to_f16_rne((float)((double)acc * sc));
+                }
+                if (M.n_src - c0 - h >= 0 && M.n_src - c0 - h < LT::HC) {  // the data column
+                    char* d = tile + lane / LT::RPR * LT::PITCH + (M.n_src - c0 - h) * 16 + lane % LT::RPR * (16 / LT::RPR);
+                    if constexpr (F64) *(double*)d = dv;
+                    else *(uint16_t*)d = f32_to_f16_rne((float)dv);
+                }
+                wave_lds_sync();
+                uint4* dst = dst0 + (size_t)(q - 1) * (F64 ? 512 : 128) + h;
+#pragma unroll
+                for (int t = lane; t < LT::NRUN * 8; t += 64)
+                    store_nt(&dst[(t >> 3) * 16 + (t & 7)], *(const uint4*)(tile + (t >> 3) * LT::PITCH + (t & 7) * 16));
+                wave_lds_sync();
+            }
         }
     }
 }
 
-int launch_build_lb_b(hipStream_t s, const BatchDev& bd, int max_rows, int max_nsup, int mixed, int cbw)
+int launch_build_lb_b(hipStream_t s, const BatchDev& bd, int max_rows, int mixed)
 {
-    if (max_rows <= 0 || max_nsup <= 0) return 0;
+    if (max_rows <= 0) return 0;
     const int max_nkt = (max_rows + TS - 1) / TS;
     const size_t esz = mixed ? 4 : 8;
     // padded tap table when it fits in 32 KB, else the compact PSF (bounds tested everywhere)
@@ -1052,15 +988,14 @@ int launch_build_lb_b(hipStream_t s, const BatchDev& bd, int max_rows, int max_n
     }
     const size_t tab_bytes = ((size_t)trows * tpc * esz + 15) / 16 * 16;
     if (tab_bytes > 64 * 1024) return -1;  // PSF beyond the LDS budget
-    const size_t tile_bytes = (size_t)TS * (cbw / 2) * (mixed ? 2 : 8) + (mixed ? TS / 4 : TS) * 16;  // + 16 B a run
-    const int nbw = (int)((bd.s_cell + 32) / 32 + 3) / 4 * 4;  // column bitmap words (16-byte multiple)
-    const size_t lds = tab_bytes + 4 * 64 * (mixed ? sizeof(LbEnt<float>) : sizeof(LbEnt<double>)) + (size_t)nbw * 4 + tile_bytes;
     if (mixed) {
+        const size_t lds = tab_bytes + 4 * (64 * sizeof(LbEnt<float>) + LbTile<float>::BYTES);
         allow_big_lds((const void*)k_build_lb_b<float>);
-        hipLaunchKernelGGL(k_build_lb_b<float>, dim3(max_nkt, bd.B), dim3(256), lds, s, bd, (int)tab_bytes, toff, tpc, trows, nbw);
+        hipLaunchKernelGGL(k_build_lb_b<float>, dim3(max_nkt, bd.B), dim3(256), lds, s, bd, (int)tab_bytes, toff, tpc, trows);
     } else {
+        const size_t lds = tab_bytes + 4 * (64 * sizeof(LbEnt<double>) + LbTile<double>::BYTES);
         allow_big_lds((const void*)k_build_lb_b<double>);
-        hipLaunchKernelGGL(k_build_lb_b<double>, dim3(max_nkt, bd.B), dim3(256), lds, s, bd, (int)tab_bytes, toff, tpc, trows, nbw);
+        hipLaunchKernelGGL(k_build_lb_b<double>, dim3(max_nkt, bd.B), dim3(256), lds, s, bd, (int)tab_bytes, toff, tpc, trows);
     }
     return 0;
 }
@@ -1126,131 +1061,206 @@ __device__ __forceinline__ bool syrk_tile(int ncb, int& I, int& J)
     return I < ncb && J <= I;
 }
 
+// Loads of a column block's strips of one chunk, all issued whatever the mask holds, so that the loads
+// behind them can be counted and stay in flight: a strip that is absent gets an offset past the buffer
+// resource's `bytes` and reads zero without touching memory.
+#define NO_STRIP 0x40000000
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t strips_rsrc(const void* pool, unsigned first, int strip_bytes, int nstrip)
+{
+    return __builtin_amdgcn_make_buffer_rsrc((char*)pool + (size_t)first * strip_bytes, 0, strip_bytes * nstrip, 0x00020000);
+}
+// byte offset of strip a (asked in order, `next` from 0), or NO_STRIP
+__device__ __forceinline__ int strip_off(unsigned mask, int a, int strip_bytes, int& next)
+{
+    const bool has = mask >> a & 1;
+    const int o = has ? next : NO_STRIP;
+    next += has ? strip_bytes : 0;
+    return o;
+}
+__device__ __forceinline__ u32x4_t load_strip(__amdgpu_buffer_rsrc_t rs, int off) { return __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0); }
+
+// The chunks k0 .. k0 + SYRK_LIST - 1 holding strips of both column blocks I and J, in order, as
+// {first strip of I's, of J's (slots in the pool), masks I | J << 8, chunk}; returns how many.  Called by
+// the 256 threads of a workgroup; `list` may be read after it and rewritten after a barrier.
+#define SYRK_LIST 512
+__device__ __forceinline__ int chunk_list(const BatchDev& bd, const ItemMeta& M, int I, int J, int k0, uint4* list, int* cnt)
+{
+    const unsigned* sI = bd.sup + M.sup_off + (size_t)I * M.nkt;
+    const unsigned* sJ = bd.sup + M.sup_off + (size_t)J * M.nkt;
+    const int* bb = bd.bbase + M.bb_off;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    unsigned e[2], f[2];
+    unsigned long long bal[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {  // group g = w + 4 u: chunks k0 + 64 g ..
+        const int k = k0 + 64 * (w + 4 * u) + lane;
+        e[u] = k < M.nkt ? sI[k] : 0u;
+        f[u] = k < M.nkt ? sJ[k] : 0u;
+        bal[u] = __ballot(e[u] && f[u]);
+        if (lane == 0) cnt[w + 4 * u] = __popcll(bal[u]);
+    }
+    __syncthreads();
+    int n = 0, off[2] = {0, 0};
+#pragma unroll
+    for (int g = 0; g < 8; g++) {
+        if (g == w) off[0] = n;
+        if (g == w + 4) off[1] = n;
+        n += cnt[g];
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int k = k0 + 64 * (w + 4 * u) + lane;
+        if (e[u] && f[u]) {
+            const unsigned b = (unsigned)bb[k];
+            list[off[u] + __popcll(bal[u] & ((1ull << lane) - 1ull))] =
+                make_uint4(b + (e[u] >> 8), b + (f[u] >> 8), (e[u] & 255u) | (f[u] & 255u) << 8, (unsigned)k);
+        }
+    }
+    __syncthreads();
+    return n;
+}
+
 // ------------------------------------------------------------------------------------------------
 // F = Lb^T C Lb, FP64 MFMA (v_mfma_f64_16x16x4f64; accumulator register v of lane l holds
-// D[l/16 + 4v][l%16] on gfx950).  One workgroup per lower tile; only chunks holding both blocks.
+// D[l/16 + 4v][l%16] on gfx950).  One workgroup per lower 64 x 64 tile; only chunks with strips in both
+// blocks, and of their 4 x 4 pairs of 16-column strips only those held (a chunk's rows reach 33 strips on
+// the 200 x 200 / 60 x 60 workload, 12.3 blocks of 64 columns: 44 % of the blocks' products).  Wave w takes
+// rows 16 w .. 16 w + 15 of every chunk for the whole tile, straight from the pool into operand registers
+// (a lane's 16 bytes are two rows of its column), so there is no staging and no barrier; its second
+// half's loads and the next chunk's first half's are in flight during the products.  The four waves'
+// sums are added in a fixed order at the end.  100 items of the workload: 44.9 ms on whole 64-blocks
+// staged in LDS, now 17.9 (10.2 ms of MFMA issue; 104 GB from beyond the L2s, 5.8 TB/s); one item 1.69 ->
+// 0.5 ms, one of 900 columns 0.27 -> 0.08.
 // ------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_syrk_f64_b(BatchDev bd)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) k_syrk_f64_b(BatchDev bd)
 {
-    __shared__ double As[TS][LDSP];
-    __shared__ double Bs[TS][LDSP];
-    extern __shared__ unsigned long long cmask[];  // chunks holding both blocks, 64 a word
+    __shared__ uint4 list[SYRK_LIST];
+    __shared__ int cnt[8];
+    __shared__ double red[2][TS * TS];
     const int item = blockIdx.y;
     const ItemMeta& M = bd.meta[item];
     if (!M.valid) return;
     int I, J;
     if (!syrk_tile(M.ncb, I, J)) return;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int wr = w >> 1, wc = w & 1;
-    const double* pool = (const double*)bd.lb + M.lb_off;
-    const double* cvec = bd.cvec + M.cvec_off;
-    const unsigned* nz = bd.nz + M.nz_off;
-    const int* bb = bd.bbase + M.bb_off;
-    const int nwd = (M.nkt + 63) >> 6;
-    for (int q = w; q < nwd; q += 4) {
-        const int k = 64 * q + lane;
-        bool b = false;
-        if (k < M.nkt) {
-            const unsigned* m = nz + (size_t)k * M.ncbw;
-            b = mask_has(m, I) && mask_has(m, J);
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool dg = I == J;
+    // rows 16 w .. of a strip: 128 16-byte pieces from 128 w on, half h of them 64
+    const double* const pool = (const double*)bd.lb + M.lb_off;
+    const int vo = (128 * w + lane) * 16;
+    const double2_t* const cvec = (const double2_t*)(bd.cvec + M.cvec_off) + 8 * w + (lane >> 4);
+    double4_t acc[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[a][c] = (double4_t){0, 0, 0, 0};
+    for (int k0 = 0; k0 < M.nkt; k0 += SYRK_LIST) {
+        const int n = chunk_list(bd, M, I, J, k0, list, cnt);
+        double2_t A[2][4], Bq[2][4], C[2];
+        unsigned mk = 0;
+        auto entry = [&](int i) {
+            const uint4 v = list[i];
+            return make_uint4((unsigned)__builtin_amdgcn_readfirstlane((int)v.x), (unsigned)__builtin_amdgcn_readfirstlane((int)v.y),
+                              (unsigned)__builtin_amdgcn_readfirstlane((int)v.z), (unsigned)__builtin_amdgcn_readfirstlane((int)v.w));
+        };
+        auto load = [&](const uint4& e, int h) {
+            const __amdgpu_buffer_rsrc_t sa = strips_rsrc(pool, e.x, 8192, 4), sb = strips_rsrc(pool, e.y, 8192, 4);
+            C[h] = cvec[(size_t)e.w * 32 + 4 * h];
+            int na = 0, nb = 0;
+#pragma unroll
+            for (int a = 0; a < 4; a++) A[h][a] = __builtin_bit_cast(double2_t, load_strip(sa, vo + 1024 * h + strip_off(e.z, a, 8192, na)));
+#pragma unroll
+            for (int c = 0; c < 4; c++) Bq[h][c] = __builtin_bit_cast(double2_t, load_strip(sb, vo + 1024 * h + strip_off(e.z, 8 + c, 8192, nb)));
+        };
+        auto mul = [&](int h) {
+            double2_t B[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) B[c] = Bq[h][c] * C[h];
+#pragma unroll
+            for (int a = 0; a < 4; a++)
+                if (mk >> a & 1)
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+                        if ((mk >> (8 + c) & 1) && !(dg && c > a)) {
+                            acc[a][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[h][a].x, B[c].x, acc[a][c], 0, 0, 0);
+                            acc[a][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[h][a].y, B[c].y, acc[a][c], 0, 0, 0);
+                        }
+        };
+        if (n) {
+            uint4 e = entry(0);
+            load(e, 0);
+            __builtin_amdgcn_sched_barrier(0);  // in this order, as in the loop: the waits count them
+            load(e, 1);
+            for (int i = 0; i < n; i++) {  // (after the last chunk the loads repeat it, for a fixed number in flight)
+                mk = e.z;
+                e = entry(min(i + 1, n - 1));
+                mul(0);
+                __builtin_amdgcn_sched_barrier(0);
+                load(e, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                mul(1);
+                __builtin_amdgcn_sched_barrier(0);
+                load(e, 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
-        const unsigned long long bal = __ballot(b);
-        if (lane == 0) cmask[q] = bal;
+        __syncthreads();  // the list is rewritten
     }
+    // ((w0 + w2) + (w1 + w3)); element (a, c, v) of a lane at ((a * 4 + c) * 4 + v) * 64 + lane
+    auto put = [&](double* d) {
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) d[((a * 4 + c) * 4 + v) * 64 + lane] = acc[a][c][v];
+    };
+    auto add = [&](const double* d) {
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[a][c][v] += d[((a * 4 + c) * 4 + v) * 64 + lane];
+    };
+    if (w >= 2) put(red[w - 2]);
     __syncthreads();
-    double4_t acc[2][2];
+    if (w < 2) add(red[w]);
+    if (w == 1) put(red[1]);
+    __syncthreads();
+    if (w) return;
+    add(red[1]);
+    double* F = (bd.Fraw ? bd.Fraw : bd.F) + M.f_off;
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int a = 0; a < 4; a++)
 #pragma unroll
-        for (int c = 0; c < 2; c++) acc[a][c] = (double4_t){0, 0, 0, 0};
-    // the next chunk after k holding both blocks (M.nkt if none)
-    auto next = [&](int k) {
-        ++k;
-        for (int q = k >> 6; q < nwd; q++) {
-            unsigned long long v = cmask[q];
-            if (q == (k >> 6)) v &= ~0ULL << (k & 63);
-            if (v) return 64 * q + __builtin_ctzll(v);
-        }
-        return M.nkt;
-    };
-    // the next chunk's blocks and weights are loaded into registers while this one is multiplied:
-    // thread element i is e = tid + 256 i (row kk = e >> 6 = tid / 64 + 4 i, column tid % 64)
-    double ra[16], rb[16], rc[16];
-    auto load = [&](int kt) {
-        const unsigned* m = nz + (size_t)kt * M.ncbw;
-        const double* Ab = pool + (size_t)(bb[kt] + mask_rank(m, I)) * TS * TS;
-        const double* Bb = pool + (size_t)(bb[kt] + mask_rank(m, J)) * TS * TS;
-        const double* cv = cvec + (size_t)kt * TS;
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            ra[i] = Ab[tid + 256 * i];
-            rb[i] = Bb[tid + 256 * i];
-            rc[i] = cv[(tid >> 6) + 4 * i];
-        }
-    };
-    int kt = next(-1);
-    if (kt < M.nkt) load(kt);
-    while (kt < M.nkt) {
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int kk = (tid >> 6) + 4 * i, ii = tid & 63;
-            As[kk][ii] = ra[i];
-            Bs[kk][ii] = rb[i] * rc[i];
-        }
-        __syncthreads();
-        const int nk = next(kt);
-        if (nk < M.nkt) load(nk);
-        kt = nk;
-#pragma unroll 4
-        for (int kk = 0; kk < TS; kk += 4) {
-            const int kq = kk + (lane >> 4);
-            double a0 = As[kq][wr * 32 + (lane & 15)];
-            double a1 = As[kq][wr * 32 + 16 + (lane & 15)];
-            double b0 = Bs[kq][wc * 32 + (lane & 15)];
-            double b1 = Bs[kq][wc * 32 + 16 + (lane & 15)];
-            acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-            acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
-        }
-    }
-    double* C = bd.F + M.f_off + (size_t)I * TS * M.ldN + (size_t)J * TS;
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-        for (int c = 0; c < 2; c++)
+        for (int c = 0; c < 4; c++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const int rr = wr * 32 + a * 16 + (lane >> 4) + 4 * v;
-                const int cc = wc * 32 + c * 16 + (lane & 15);
-                C[(size_t)rr * M.ldN + cc] = acc[a][c][v];
+                const int r = I * TS + a * 16 + (lane >> 4) + 4 * v, q = J * TS + c * 16 + (lane & 15);
+                F[(size_t)r * M.ldN + q] = r > M.n_src ? (r == q ? 1.0 : 0.0) : acc[a][c][v];  // identity beyond the data row
             }
 }
 
-void launch_syrk_f64_b(hipStream_t s, const BatchDev& bd, int max_ncb, int max_nkt)
+void launch_syrk_f64_b(hipStream_t s, const BatchDev& bd, int max_ncb)
 {
-    hipLaunchKernelGGL(k_syrk_f64_b, dim3(syrk_grid(max_ncb), bd.B), dim3(256), (size_t)((max_nkt + 63) / 64) * 8, s, bd);
+    hipLaunchKernelGGL(k_syrk_f64_b, dim3(syrk_grid(max_ncb), bd.B), dim3(256), 0, s, bd);
 }
 
 // ------------------------------------------------------------------------------------------------
-// F32 = Lb^T Lb on the mixed path: one FP16 pool of sqrt(c) s16-scaled rows in k4-interleaved
-// 64 x 128 blocks, v_mfma_f32_16x16x32_f16 accumulated in FP32, scaled back by s16^-2 (exact) at
-// the store.  One workgroup per 128x128 lower tile of F; wave (wr, wc) computes the 64x64 quadrant
-// (wr, wc).  A operand lane l holds A[i = l%16][8 consecutive k], B the same with j; accumulator
-// register v of lane l holds D[4*(l/16) + v][l%16].  The next chunk's two blocks are loaded into
-// registers while the current chunk is multiplied from LDS.
+// F32 = Lb^T Lb on the mixed path: one FP16 pool of sqrt(c) s16-scaled rows in strips of 16 columns,
+// v_mfma_f32_16x16x32_f16 accumulated in FP32, scaled back by s16^-2 (exact) at the store.  One
+// workgroup per 128 x 128 lower tile of F.  A operand lane l holds A[i = l%16][8 consecutive k], B the
+// same with j; accumulator register v of lane l holds D[4*(l/16) + v][l%16].  Only the strips a chunk
+// holds are read (33 of 16 columns a chunk on the 200 x 200 / 60 x 60 workload against 8.5 blocks of
+// 128) and multiplied.  As in the FP64 kernel the operands come straight from the pool into registers,
+// SYRK_D chunks ahead, with no staging and no barrier: wave (kh, jh) takes rows 32 kh .. of every chunk for
+// the tile's columns 64 jh .. (16-byte loads: a wave's load occupies the L1 for 16 cycles whatever its
+// width, and four waves of 16 rows with 8-byte ones took 14.4 ms).  The two row halves' sums are added
+// at the end, each wave finishing 64 x 64.  256 items of the workload: 15.3 ms on whole 128-blocks staged
+// in LDS (114 GB from beyond the L2s), 15.6 with the strips staged there, now 10.1 (36 GB; 7 of them are
+// issue: the masks' offsets and branches).
 // ------------------------------------------------------------------------------------------------
 #define SCB 128  // column-block width of the mixed path
-#define BP2 544  // LDS elements per k-group: 128 columns x 4 k + 32, so the four lane groups of a
-                 // 64-bit operand read fall on alternating bank halves
-__device__ __forceinline__ f16x8_t lds_k8(const uint16_t* arr, int g, int i)
-{
-    const uint2 a = *(const uint2*)&arr[g * BP2 + i * 4];
-    const uint2 b = *(const uint2*)&arr[(g + 1) * BP2 + i * 4];
-    return __builtin_bit_cast(f16x8_t, make_uint4(a.x, a.y, b.x, b.y));
-}
-
 __device__ __forceinline__ double item_lambda(const BatchDev& bd, int item) { return bd.lam ? bd.lam[item] : bd.lambda; }
 
 // R entry (r, c), c <= r, of the banded curvature tiles (reference order, |r - c| within the band)
@@ -1265,160 +1275,120 @@ __device__ __forceinline__ double rget(const BatchDev& bd, int item, int r, int 
     return *rtile(bd, bd.meta[bd.rrep[item]], r, c);
 }
 
-// F's preparation, fused into the FP16 SYRK's store of tile (I, J): scale back, F += lambda R over
-// the source block (R is held in the reference order: internal indices map through pisrc), the data
-// row n kept with a large pivot (the refined solve never reads it), identity beyond n and the FP64
-// diagonal into Fdiag.  A diagonal tile's upper half gets the same symmetric formula.  The tiles go to
-// Ff32 (F as formed, which the refinement residual reads); the Cholesky kernels that touch a block
-// first (the first part's diagonal and panel kernels, the first strip and trailing updates) read it
-// there and write the factor buffer F32.  Wave (wr, wc) holds quadrant (wr, wc).
-__device__ __forceinline__ void syrk_f16_store(const BatchDev& bd, const ItemMeta& M, int item, int I, int J,
-                                               const float4_t (&acc)[4][4])
+// The FP16 SYRK's store: scaled back, the data row n kept with a large pivot (the refined solve never
+// reads it), identity beyond n.  k_add_reg_b then adds lambda R.  The tiles go to Ff32 (F as formed); the
+// Cholesky kernels that touch a block first (the first part's diagonal and panel kernels, the first
+// strip and trailing updates) read it there and write the factor buffer F32.  A diagonal 64-tile is
+// held whole (the refinement residual reads its upper half).  acc: 64 rows r0 .., 64 columns c0 ..
+__device__ __forceinline__ void syrk_f16_store(const BatchDev& bd, const ItemMeta& M, int r0, int c0, const float4_t (&acc)[4][4])
 {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int wr = w >> 1, wc = w & 1;
+    const int lane = threadIdx.x & 63;
     const float unscale = (float)(1.0 / (bd.s16 * bd.s16));
     const int ld = M.ldN, n = M.n_src;
-    const double lam = item_lambda(bd, item);
-    const int* pis = bd.pisrc + item * bd.s_cell;
-    double* fdiag = bd.vec + M.vec_off + 3 * (size_t)ld;
-    float* C = bd.Ff32 + M.f_off + (size_t)I * SCB * ld + (size_t)J * SCB;
-    const int r0 = I * SCB + wr * 64 + 4 * (lane >> 4), c0 = J * SCB + wc * 64 + (lane & 15);
+    float* C = bd.Ff32 + M.f_off;
+    r0 += 4 * (lane >> 4);
+    c0 += lane & 15;
 #pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const int cg = c0 + c * 16;
-        const int pb = cg < n ? pis[cg] : -1;
+    for (int c = 0; c < 4; c++)
 #pragma unroll
         for (int a = 0; a < 4; a++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const int r = r0 + a * 16 + v;
+                const int r = r0 + a * 16 + v, cg = c0 + c * 16;
                 float x = acc[a][c][v] * unscale;
-                if (r < n && cg < n) {
-                    const int pa = pis[r];
-                    const int hi = pa > pb ? pa : pb, lo = pa > pb ? pb : pa;
-                    if ((hi >> 6) - (lo >> 6) <= M.bwb) x = (float)((double)x + lam * rget(bd, item, hi, lo));
-                    if (r == cg) fdiag[r] = (double)x;
-                } else if (r > n || cg > n) {
-                    x = (r == cg) ? 1.0f : 0.0f;
-                } else if (r == cg) {
-                    x = 1e30f;  // (n, n); the rest of row n (D) is kept
-                }
-                __builtin_nontemporal_store(x, &C[(size_t)(r - I * SCB) * ld + (cg - J * SCB)]);
+                if (r > n || cg > n) x = (r == cg) ? 1.0f : 0.0f;
+                else if (r == n && cg == n) x = 1e30f;  // the rest of row n (D) is kept
+                __builtin_nontemporal_store(x, &C[(size_t)r * ld + cg]);
             }
-    }
 }
 
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 4))) k_syrk_f16_b(BatchDev bd)
+#define SYRK_D 2
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) k_syrk_f16_b(BatchDev bd)
 {
-    extern __shared__ __attribute__((aligned(16))) uint16_t lds2[];  // A, B: 16 x BP2 each
+    __shared__ uint4 list[SYRK_LIST];
+    __shared__ int cnt[8];
+    __shared__ float4_t red[4][16 * 64];
     const int item = blockIdx.y;
     const ItemMeta& M = bd.meta[item];
     if (!M.valid) return;
     int I, J;
     if (!syrk_tile(M.ncb, I, J)) return;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int wr = w >> 1, wc = w & 1;
-    const size_t bsz = (size_t)TS * SCB;
-    const uint16_t* pool = (const uint16_t*)bd.lb + M.lb_off;
-    const unsigned* nz = bd.nz + M.nz_off;
-    const int* bb = bd.bbase + M.bb_off;
-    const int nkt = M.nkt, ncbw = M.ncbw;
-    uint16_t* const as = lds2;
-    uint16_t* const bs = lds2 + 16 * BP2;
-    const bool dg = I == J;  // a diagonal tile reads its one block once, as both operands
-    const uint16_t* const bsrc = dg ? as : bs;
-    // thread piece h (of 4) of every block: 16 bytes at element (tid + 256 h) * 8
-    const int e0 = tid * 8;
-    const int o0 = (e0 >> 9) * BP2 + (e0 & 511);                    // pieces h = 0..3 are 2048
-    const int o1 = ((e0 + 2048) >> 9) * BP2 + ((e0 + 2048) & 511);  // elements apart: 4 k-groups
-    const int o2 = ((e0 + 4096) >> 9) * BP2 + ((e0 + 4096) & 511);
-    const int o3 = ((e0 + 6144) >> 9) * BP2 + ((e0 + 6144) & 511);
-    // the chunks holding both blocks as a bit mask in LDS (64 chunks a word, one ballot each), so
-    // that finding the next one is a word test rather than a scan of the chunks' supports
-    unsigned long long* const cmask = (unsigned long long*)(lds2 + 32 * BP2);
-    const int nwd = (nkt + 63) >> 6;
-    for (int q = w; q < nwd; q += 4) {
-        const int k = 64 * q + lane;
-        bool b = false;
-        if (k < nkt) {
-            const unsigned* m = nz + (size_t)k * ncbw;
-            b = mask_has(m, I) && mask_has(m, J);
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kh = w >> 1, jh = w & 1;
+    // rows 32 kh .. of a strip: its 16-byte pieces 64 kh ..
+    const uint16_t* const pool = (const uint16_t*)bd.lb + M.lb_off;
+    const int vo = (64 * kh + lane) * 16;
+    const unsigned rowsel = I == J && jh ? 0xf0u : 0xffu;  // (above the diagonal: not needed)
+    float4_t acc[8][4];
+#pragma unroll
+    for (int a = 0; a < 8; a++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) acc[a][c] = (float4_t){0, 0, 0, 0};
+    for (int k0 = 0; k0 < M.nkt; k0 += SYRK_LIST) {
+        const int n = chunk_list(bd, M, I, J, k0, list, cnt);
+        f16x8_t A[SYRK_D][8], B[SYRK_D][4];
+        unsigned mk[SYRK_D];  // strips of the rows, of the wave's 64 columns << 8
+        auto load = [&](int i, int s) {
+            const uint4 v = list[i];
+            const unsigned m = (unsigned)__builtin_amdgcn_readfirstlane((int)v.z);
+            const unsigned mj = m >> (8 + 4 * jh) & 15u, mi = mj ? m & rowsel : 0u;
+            const __amdgpu_buffer_rsrc_t sa = strips_rsrc(pool, (unsigned)__builtin_amdgcn_readfirstlane((int)v.x), 2048, 8);
+            const __amdgpu_buffer_rsrc_t sb = strips_rsrc(pool, (unsigned)__builtin_amdgcn_readfirstlane((int)v.y), 2048, 8);
+            int na = 2048 * __popc(m & 255u & ~rowsel), nb = jh ? 2048 * __popc(m >> 8 & 15u) : 0;
+            mk[s] = mi;
+#pragma unroll
+            for (int a = 0; a < 8; a++) A[s][a] = __builtin_bit_cast(f16x8_t, load_strip(sa, vo + strip_off(mi, a, 2048, na)));
+#pragma unroll
+            for (int c = 0; c < 4; c++) B[s][c] = __builtin_bit_cast(f16x8_t, load_strip(sb, vo + strip_off(mj, c, 2048, nb)));
+        };
+        // SYRK_D chunks at a time; past the last one the loads repeat it and the products are left out, so
+        // that the number of loads behind each product is fixed
+        if (n) {
+#pragma unroll
+            for (int s = 0; s < SYRK_D; s++) {
+                load(min(s, n - 1), s);
+                __builtin_amdgcn_sched_barrier(0);  // in this order, as in the loop: the waits count them
+            }
+            for (int i0 = 0; i0 < n; i0 += SYRK_D)
+#pragma unroll
+                for (int s = 0; s < SYRK_D; s++) {
+                    const unsigned m = i0 + s < n ? mk[s] : 0u;
+#pragma unroll
+                    for (int a = 0; a < 8; a++)
+                        if (m >> a & 1)
+#pragma unroll
+                            for (int c = 0; c < 4; c++)
+                                acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[s][a], B[s][c], acc[a][c], 0, 0, 0);
+                    load(min(i0 + s + SYRK_D, n - 1), s);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
         }
-        const unsigned long long bal = __ballot(b);
-        if (lane == 0) cmask[q] = bal;
+        __syncthreads();  // the list is rewritten
     }
-    __syncthreads();
-    // the next chunk after k holding both blocks (nkt if none)
-    auto next = [&](int k) {
-        ++k;
-        for (int q = k >> 6; q < nwd; q++) {
-            unsigned long long v = cmask[q];
-            if (q == (k >> 6)) v &= ~0ULL << (k & 63);
-            if (v) return 64 * q + __builtin_ctzll(v);
-        }
-        return nkt;
-    };
-#define SYRK_LOAD(kk_, A0, A1, A2, A3, B0, B1, B2, B3)                                                  \
-    {                                                                                                    \
-        const unsigned* m_ = nz + (size_t)(kk_) * ncbw;                                                  \
-        const uint4* a_ = (const uint4*)(pool + (size_t)(bb[kk_] + mask_rank(m_, I)) * bsz) + tid;       \
-        A0 = a_[0]; A1 = a_[256]; A2 = a_[512]; A3 = a_[768];                                            \
-        if (!dg) {                                                                                       \
-            const uint4* b_ = (const uint4*)(pool + (size_t)(bb[kk_] + mask_rank(m_, J)) * bsz) + tid;   \
-            B0 = b_[0]; B1 = b_[256]; B2 = b_[512]; B3 = b_[768];                                        \
-        }                                                                                                \
-    }
-#define SYRK_STAGE(A0, A1, A2, A3, B0, B1, B2, B3)                                                       \
-    {                                                                                                    \
-        __syncthreads();                                                                                 \
-        *(uint4*)&as[o0] = A0; *(uint4*)&as[o1] = A1; *(uint4*)&as[o2] = A2; *(uint4*)&as[o3] = A3;      \
-        if (!dg) { *(uint4*)&bs[o0] = B0; *(uint4*)&bs[o1] = B1; *(uint4*)&bs[o2] = B2; *(uint4*)&bs[o3] = B3; } \
-        __syncthreads();                                                                                 \
-    }
-    float4_t acc[4][4];
+    // wave (kh, jh) finishes the tile's rows 64 kh .. of its columns: its own sums and wave (1 - kh, jh)'s
+    float4_t o[4][4];
 #pragma unroll
     for (int a = 0; a < 4; a++)
 #pragma unroll
-        for (int c = 0; c < 4; c++) acc[a][c] = (float4_t){0, 0, 0, 0};
-    auto mma = [&]() {
-#pragma unroll
-        for (int k0 = 0; k0 < TS; k0 += 32) {
-            const int g = (k0 >> 2) + 2 * (lane >> 4);
-            f16x8_t av[4], bv[4];
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                av[t] = lds_k8(as, g, wr * 64 + t * 16 + (lane & 15));
-                bv[t] = lds_k8(bsrc, g, wc * 64 + t * 16 + (lane & 15));
-            }
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int c = 0; c < 4; c++) acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[a], bv[c], acc[a][c], 0, 0, 0);
+        for (int c = 0; c < 4; c++) {
+            o[a][c] = kh ? acc[4 + a][c] : acc[a][c];
+            red[w][(a * 4 + c) * 64 + lane] = kh ? acc[a][c] : acc[4 + a][c];
         }
-    };
-    // the next chunk's blocks are loaded into registers while this one is multiplied (loading two
-    // chunks ahead needs 176 registers, two waves per SIMD, and took 23.3 ms against 17.2)
-    uint4 pa0, pa1, pa2, pa3, pb0, pb1, pb2, pb3;
-    int kt = next(-1);
-    if (kt < nkt) SYRK_LOAD(kt, pa0, pa1, pa2, pa3, pb0, pb1, pb2, pb3);
-    while (kt < nkt) {
-        SYRK_STAGE(pa0, pa1, pa2, pa3, pb0, pb1, pb2, pb3);
-        const int nk = next(kt);
-        if (nk < nkt) SYRK_LOAD(nk, pa0, pa1, pa2, pa3, pb0, pb1, pb2, pb3);
-        mma();
-        kt = nk;
-    }
-#undef SYRK_LOAD
-#undef SYRK_STAGE
-    syrk_f16_store(bd, M, item, I, J, acc);
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float4_t t = red[w ^ 2][(a * 4 + c) * 64 + lane];
+            o[a][c] = kh ? t + o[a][c] : o[a][c] + t;
+        }
+    if (I == J && jh > kh) return;  // above the diagonal
+    syrk_f16_store(bd, M, I * SCB + 64 * kh, J * SCB + 64 * jh, o);
 }
 
-void launch_syrk_f16_b(hipStream_t s, const BatchDev& bd, int max_ncb, int max_nkt)
+void launch_syrk_f16_b(hipStream_t s, const BatchDev& bd, int max_ncb)
 {
-    const size_t lds = (size_t)2 * 16 * BP2 * sizeof(uint16_t) + (size_t)((max_nkt + 63) / 64) * 8;
-    allow_big_lds((const void*)k_syrk_f16_b);
-    hipLaunchKernelGGL(k_syrk_f16_b, dim3(syrk_grid(max_ncb), bd.B), dim3(256), lds, s, bd);
+    hipLaunchKernelGGL(k_syrk_f16_b, dim3(syrk_grid(max_ncb), bd.B), dim3(256), 0, s, bd);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1559,50 +1529,71 @@ void launch_curvature_b(hipStream_t s, const BatchDev& bd, int max_cells, int ma
     hipLaunchKernelGGL(k_curvature_b, dim3((n + 255) / 256, bd.B), dim3(256), 0, s, bd);
 }
 
-// FP64 path: F_lower += lambda R over the n x n source block; row n (the data row D^T | d^T C d of
-// the augmented factorization) is kept, rows > n are identity.  (The mixed path does this in the
-// FP16 SYRK's epilogue, syrk_f16_store.)
-__global__ void __launch_bounds__(256) k_prep_f_b(BatchDev bd)
+// regparam optimisation: F's lower tiles from F as formed (Fraw), for the next lambda
+__global__ void __launch_bounds__(256) k_copy_f_b(BatchDev bd)
 {
     const int item = blockIdx.y;
     const ItemMeta& M = bd.meta[item];
     if (!M.valid) return;
-    const int ld = M.ldN, n = M.n_src, nb = ld / TS;
+    const int nb = M.ldN / TS;
     if ((int)blockIdx.x >= nb * (nb + 1) / 2) return;
     int I, J;
     tri_decode(blockIdx.x, I, J);
-    double* F = bd.F + M.f_off;
-    const double* F0 = bd.Fraw ? bd.Fraw + M.f_off : F;  // out of place when F as formed is kept
-    const int* pis = bd.pisrc + item * bd.s_cell;
+    const size_t o = M.f_off + (size_t)I * TS * M.ldN + (size_t)J * TS;
+#pragma unroll
+    for (int e = 2 * threadIdx.x; e < TS * TS; e += 512) {
+        const size_t t = o + (size_t)(e >> 6) * M.ldN + (e & 63);
+        *(double2_t*)&bd.F[t] = *(const double2_t*)&bd.Fraw[t];
+    }
+}
+
+// F += lambda R.  R couples a cell with itself and the cells one and two away along each axis, so a
+// thread takes a cell's five pairs that lie ahead of it: a pass over those entries instead of one over F
+// that gathered an R entry for each of its own (FP16 SYRK's store 17.7 -> 13.8 ms of the kernel per 256
+// items of 3600 cells, the FP64 pass 2.45 ms per 100).  R is held in the reference order, F in the
+// internal one.  FP32: the diagonal 64-tiles' upper halves too, and the diagonal in FP64 into Fdiag.
+template <typename T>
+__global__ void __launch_bounds__(256) k_add_reg_b(BatchDev bd)
+{
+    const int item = blockIdx.y;
+    const ItemMeta& M = bd.meta[item];
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (!M.valid || c >= M.snx * M.sny) return;
+    const int* sidx = bd.sidx + item * bd.s_cell;
+    const int* tix = bd.tix + item * bd.s_cell;
+    if (sidx[c] < 0) return;
+    const int i = c / M.sny, j = c - i * M.sny;
+    T* F = (sizeof(T) == 8 ? (T*)bd.F : (T*)bd.Ff32) + M.f_off;
+    double* fdiag = bd.vec + M.vec_off + 3 * (size_t)M.ldN;
     const double lam = item_lambda(bd, item);
-    // 16 elements per thread, unrolled so that their gathers (pisrc, R tile, F) are in flight together
-#pragma unroll 8
-    for (int e = threadIdx.x; e < TS * TS; e += 256) {
-        const int rr = e >> 6, cc = e & 63;
-        const int r = I * TS + rr, c = J * TS + cc;
-        if (c <= r) {
-            const size_t t = (size_t)r * ld + c;
-            if (r < n) {
-                // R is held in the reference order: F's internal indices map through pisrc
-                const int a = pis[r], b = pis[c];
-                const int hi = a > b ? a : b, lo = a > b ? b : a;
-                const double rv = ((hi >> 6) - (lo >> 6) <= M.bwb) ? rget(bd, item, hi, lo) : 0.0;
-                F[t] = F0[t] + lam * rv;
-            } else if (r > n) {
-                F[t] = (r == c) ? 1.0 : 0.0;
-            } else {
-                F[t] = F0[t];  // the data row
-            }
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+        const int di = k == 1 ? 1 : k == 2 ? 2 : 0, dj = k == 3 ? 1 : k == 4 ? 2 : 0;
+        if (i + di >= M.snx || j + dj >= M.sny) continue;
+        const int d = c + di * M.sny + dj;
+        if (sidx[d] < 0) continue;
+        const int pa = sidx[c], pb = sidx[d], a = tix[c], b = tix[d];
+        const int r = a > b ? a : b, q = a > b ? b : a;
+        T* f = &F[(size_t)r * M.ldN + q];
+        const T x = (T)((double)*f + lam * rget(bd, item, pa > pb ? pa : pb, pa > pb ? pb : pa));
+        *f = x;
+        if (sizeof(T) == 4) {
+            if (k == 0) fdiag[r] = (double)x;
+            else if ((r >> 6) == (q >> 6)) F[(size_t)q * M.ldN + r] = x;
         }
     }
 }
 
-void launch_prep_fr_b(hipStream_t s, const BatchDev& bd, int max_ld, int f32)
+void launch_add_reg_b(hipStream_t s, const BatchDev& bd, int max_ld, int max_cells, int f32)
 {
+    const dim3 grid((max_cells + 255) / 256, bd.B);
+    if (f32) {
+        hipLaunchKernelGGL(k_add_reg_b<float>, grid, dim3(256), 0, s, bd);
+        return;
+    }
     const int nb = max_ld / TS;
-    if (f32) return;  // the mixed path's FP16 SYRK prepares F in its epilogue
-    const unsigned g = nb * (nb + 1) / 2;
-    hipLaunchKernelGGL(k_prep_f_b, dim3(g, bd.B), dim3(256), 0, s, bd);
+    if (bd.Fraw) hipLaunchKernelGGL(k_copy_f_b, dim3(nb * (nb + 1) / 2, bd.B), dim3(256), 0, s, bd);
+    hipLaunchKernelGGL(k_add_reg_b<double>, grid, dim3(256), 0, s, bd);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -96,10 +96,10 @@ struct Ctx {
     DevBuf d_models, d_sgrid, d_srcn, d_meta, d_mats;
     // per-item work (stride s_pix / s_cell)
     DevBuf beta, map_cell, map_w, pmapped, cmapped, sidx, tix, pisrc, pidx, act_pix, counts, ucol, uval, ucnt, nevals;
-    DevBuf apre, eptr, csh, cpix, cval, nfwtab, pmask, hmask, rdup;
+    DevBuf apre, eptr, csh, cpix, cval, nfwtab, rdup;
     DevBuf key, bcnt, boff, bfill, perm;
     // pools
-    DevBuf lb, F, Ff, Fz, R, Rf, cvec, vec, nz, bbase, winv, model, out, status;  // Fz: residual partials  // Rf: R's copy for its factorization
+    DevBuf lb, F, Ff, Fz, R, Rf, cvec, vec, nz, colb, sup, bbase, winv, model, out, status;  // Fz: residual partials  // Rf: R's copy for its factorization
     DevBuf Fraw, d_lam;  // regparam optimisation: F as formed and the per-item lambda
     DevBuf agrid;        // automatic source grids: per item box and centre-ray count
     // solutions of the last call, kept on the device for qlx_get_source: per caller item a block
@@ -119,7 +119,6 @@ struct Ctx {
     bool fit_set = false;
     std::vector<int> last_wave;  // caller indices of the last wave's items, in wave order (their rays
                                  // stay in `beta` until the next evaluation)
-    std::vector<unsigned> nzh;  // host copy of the support masks (work accounting)
     std::map<int, int> chol_tuned;  // autotuned FP32 Cholesky panel (64-blocks) per padded block count
     int last_panel = 0;
     // captured factorization sequences: (stream, MatDesc array, counts, sizes, panel) -> executable
@@ -345,7 +344,7 @@ void fill_source_grid(const double* box, int snx, int sny, double* g)
 size_t stage1_bytes(size_t s_pix, size_t s_cell, size_t nsub)
 {
     const size_t U = 3 * nsub;
-    return s_pix * nsub * (16 + 12 + 24) + s_pix * U * 24 + (size_t)csc_segments(s_pix) * s_cell * 4 + s_pix * 4 * 7 + (s_pix + 1) * 12 + s_cell * 4 * 5 + 64 + s_pix * 16 + QLX_NFWTAB_DOUBLES * 8 + s_pix * QLX_MAX_CBW * 4;
+    return s_pix * nsub * (16 + 12 + 24) + s_pix * U * 24 + (size_t)csc_segments(s_pix) * s_cell * 4 + s_pix * 4 * 7 + (s_pix + 1) * 12 + s_cell * 4 * 5 + 64 + s_pix * 16 + QLX_NFWTAB_DOUBLES * 8;
 }
 
 // upper bound of the dense bytes of one item with at most ncell active source cells
@@ -564,11 +563,10 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
               c->sidx.ensure(B * s_cell * 4) && c->tix.ensure(B * s_cell * 4) && c->pisrc.ensure(B * s_cell * 4) &&
               c->pidx.ensure(B * s_pix * 4) && c->act_pix.ensure(B * s_pix * 4) &&
               c->counts.ensure((size_t)B * 16) && c->ucol.ensure(B * s_pix * U * 4) && c->uval.ensure(B * s_pix * U * 8) &&
-              c->ucnt.ensure(B * s_pix * 4) && c->nevals.ensure((size_t)B * 8) && c->key.ensure(B * s_pix * 4) &&
+              c->ucnt.ensure(B * s_pix * 4) && c->nevals.ensure((size_t)B * 16) && c->key.ensure(B * s_pix * 4) &&
               c->apre.ensure(B * (s_pix + 1) * 4) && c->eptr.ensure(B * (s_pix + 1) * 4) &&
               c->csh.ensure(B * (size_t)csc_segments(s_pix) * s_cell * 4) && c->cpix.ensure(B * s_pix * U * 4) && c->cval.ensure(B * s_pix * U * 8) &&
               c->nfwtab.ensure((size_t)B * QLX_NFWTAB_DOUBLES * 8) &&
-              c->pmask.ensure((size_t)B * s_pix * QLX_MAX_CBW * 4) && c->hmask.ensure((size_t)B * s_pix * QLX_MAX_CBW * 4) &&
               c->bcnt.ensure(B * (s_cell + 2) * 4) && c->boff.ensure(B * (s_cell + 2) * 4) && c->bfill.ensure(B * (s_cell + 2) * 4) &&
               c->perm.ensure(B * s_pix * 4) && c->model.ensure(B * s_pix * 16) && c->out.ensure((size_t)B * QLX_OUT_STRIDE * 8) &&
               c->status.ensure((size_t)B * 16) && c->agrid.ensure((size_t)B * 64) &&
@@ -622,8 +620,6 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
     bd.cpix = c->cpix.as<unsigned>();
     bd.cval = c->cval.as<double>();
     bd.nfwtab = c->nfwtab.as<double>();
-    bd.pmask = c->pmask.as<unsigned>();
-    bd.hmask = c->hmask.as<unsigned>();
     {
         // mixed-path pool entries are x = (blurred L entry) sqrt(c) or data sqrt(c), with
         // |blurred L entry| <= sum|psf| * max_r ||L_r||_1 <= 3 sum|psf| (per subpixel the 3-point
@@ -643,6 +639,7 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
     bd.bfill = c->bfill.as<int>();
     bd.perm = c->perm.as<int>();
     bd.nevals = c->nevals.as<unsigned long long>();
+    bd.npairs = bd.nevals + B;
     bd.s_pix = (long long)s_pix;
     bd.s_cell = (long long)s_cell;
     bd.meta = c->d_meta.as<ItemMeta>();
@@ -653,7 +650,7 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
     launch_fill_i32(st, bd.pmapped, 0, B * s_pix);
     launch_fill_i32(st, bd.cmapped, 0, B * s_cell);
     launch_fill_i32(st, bd.status, 0, (size_t)B * 4);
-    launch_fill_i32(st, (int*)bd.nevals, 0, (size_t)B * 2);
+    launch_fill_i32(st, (int*)bd.nevals, 0, (size_t)B * 4);
     launch_fill_f64(st, bd.out, 0.0, (size_t)B * QLX_OUT_STRIDE);
 
     timer_begin(c, "total");
@@ -706,8 +703,8 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
 
     // ---- per-item dense sizes ----
     std::vector<ItemMeta> meta(B);
-    size_t f_tot = 0, r_tot = 0, cv_tot = 0, vec_tot = 0, nz_tot = 0, bb_tot = 0, w_tot = 0;
-    int max_img = 0, max_src = 0, max_rows = 0, max_nkt = 0, max_ncb = 0, max_ld = 0, max_cells = 0, max_rtiles = 0;
+    size_t f_tot = 0, r_tot = 0, cv_tot = 0, vec_tot = 0, nz_tot = 0, col_tot = 0, sup_tot = 0, bb_tot = 0, w_tot = 0;
+    int max_img = 0, max_src = 0, max_rows = 0, max_nkt = 0, max_ncb = 0, max_ld = 0, max_cells = 0, max_rtiles = 0, max_sup = 0;
     for (int b = 0; b < B; b++) {
         ItemMeta& M = meta[b];
         memset(&M, 0, sizeof(M));
@@ -743,11 +740,12 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
         }
         M.valid = 1;
         M.keep_off = (long long)c->kept[items[b].idx].off;
-        M.cbs = mixed ? 7 : 6;  // Lb column blocks of 128 (mixed) or 64 (FP64) source pixels
+        M.cbs = mixed ? 7 : 6;  // SYRK column blocks of 128 (mixed) or 64 (FP64) source pixels
         M.ldN = (int)round_up((size_t)n_src + 1, 128);  // 128: whole tiles of the trailing Cholesky update
         M.nrows = (int)std::max<size_t>(64, round_up((size_t)n_img, 64));
         M.ncb = M.ldN >> M.cbs;
-        M.ncbw = (M.ncb + 31) / 32;
+        M.ncw = M.ldN / 32;
+        M.nsw = (M.ldN / 16 + 31) / 32;
         M.nkt = M.nrows / 64;
         M.bwb = (2 * M.snx) / 64 + 1;
         const size_t nb = M.ldN / 64;
@@ -760,7 +758,11 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
         M.vec_off = (long long)vec_tot;
         vec_tot += (size_t)QLX_VEC_SLOTS * M.ldN;
         M.nz_off = (long long)nz_tot;
-        nz_tot += (size_t)M.nkt * M.ncbw;
+        nz_tot += (size_t)M.nkt * M.nsw;
+        M.col_off = (long long)col_tot;
+        col_tot += (size_t)M.nkt * M.ncw;
+        M.sup_off = (long long)sup_tot;
+        sup_tot += (size_t)M.ncb * M.nkt;
         M.bb_off = (long long)bb_tot;
         bb_tot += M.nkt + 1;
         M.w_off = (long long)w_tot;
@@ -770,6 +772,7 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
         max_rows = std::max(max_rows, M.nrows);
         max_nkt = std::max(max_nkt, M.nkt);
         max_ncb = std::max(max_ncb, M.ncb);
+        max_sup = std::max(max_sup, M.ncb * M.nkt);
         max_ld = std::max(max_ld, M.ldN);
         max_cells = std::max(max_cells, M.snx * M.sny);
         max_rtiles = std::max(max_rtiles, (int)(nb * (M.bwb + 1)));
@@ -782,10 +785,10 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
     }
     const bool opt = S.optimize_regparam != 0 && !mixed;
     const size_t fixed_bytes = (size_t)B * stage1_bytes(s_pix, s_cell, nsub);
-    const size_t dense_bytes = f_tot * (opt ? 16 : 8) + r_tot * 16 + cv_tot * 8 + vec_tot * 8 + nz_tot * 4 + bb_tot * 4 + w_tot * 8 +
+    const size_t dense_bytes = f_tot * (opt ? 16 : 8) + r_tot * 16 + cv_tot * 8 + vec_tot * 8 + (nz_tot + col_tot + sup_tot + bb_tot) * 4 + w_tot * 8 +
                                (mixed ? f_tot / 16 : 0);
     if (B > 1 && fixed_bytes + dense_bytes > budget) return WAVE_TOO_BIG;
-    ok = c->R.ensure(r_tot * 8) && c->Rf.ensure(r_tot * 8) && c->cvec.ensure(cv_tot * 8) && c->vec.ensure(vec_tot * 8) && c->nz.ensure(nz_tot * 4) &&
+    ok = c->R.ensure(r_tot * 8) && c->Rf.ensure(r_tot * 8) && c->cvec.ensure(cv_tot * 8) && c->vec.ensure(vec_tot * 8) && c->nz.ensure(nz_tot * 4) && c->colb.ensure(col_tot * 4) && c->sup.ensure(sup_tot * 4) &&
          c->bbase.ensure(bb_tot * 4) && c->winv.ensure(w_tot * 8) && c->F.ensure(f_tot * (mixed ? 4 : 8)) &&
          (!mixed || (c->Ff.ensure(f_tot * 4) && c->Fz.ensure(f_tot / 16)));
     if (!ok) return fail(c, QLX_ERR_NOMEM, "dense buffer allocation failed (F/R)");
@@ -797,6 +800,8 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
     bd.cvec = c->cvec.as<double>();
     bd.vec = c->vec.as<double>();
     bd.nz = c->nz.as<unsigned>();
+    bd.colb = c->colb.as<unsigned>();
+    bd.sup = c->sup.as<unsigned>();
     bd.bbase = c->bbase.as<int>();
     bd.winv = c->winv.as<double>();
     HIPCHK(c, hipMemcpyAsync(c->d_meta.p, meta.data(), sizeof(ItemMeta) * B, hipMemcpyHostToDevice, st));
@@ -805,11 +810,9 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
     launch_merge_lrows_b(st, bd, max_img);
     launch_sort_rows_b(st, bd, max_img, max_src);
     launch_lcols_b(st, bd, max_img, max_src);
-    launch_row_support_b(st, bd, max_nkt);
+    launch_row_support_b(st, bd, max_nkt, max_ld, max_sup);
     launch_rdup_b(st, bd);
     HIPCHK(c, hipMemcpyAsync(counts.data(), bd.counts, (size_t)B * 16, hipMemcpyDeviceToHost, st));
-    c->nzh.resize(nz_tot);
-    HIPCHK(c, hipMemcpyAsync(c->nzh.data(), bd.nz, nz_tot * 4, hipMemcpyDeviceToHost, st));
     std::vector<int> rrep(B);
     HIPCHK(c, hipMemcpyAsync(rrep.data(), bd.rrep, (size_t)B * 4, hipMemcpyDeviceToHost, st));
     HIPCHK(c, hipStreamSynchronize(st));
@@ -851,27 +854,24 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
     HIPCHK(c, hipMemcpyAsync(c->d_mats.p, mats.data(), sizeof(MatDesc) * mats.size(), hipMemcpyHostToDevice, st));
     const int nF = (int)fm.size(), nR = (int)rm.size();
     size_t lb_tot = 0;
-    int max_nsup = 0;
     for (int b = 0; b < B; b++) {
         ItemMeta& M = meta[b];
         if (!M.valid) continue;
         M.nblk = counts[4 * b + 2];
-        M.nsup_max = counts[4 * b + 3];
         M.lb_off = (long long)lb_tot;
-        lb_tot += (size_t)M.nblk * ((size_t)64 << M.cbs);
-        max_nsup = std::max(max_nsup, M.nsup_max);
+        lb_tot += (size_t)M.nblk * 1024;  // strips of 64 x 16
     }
     if (B > 1 && fixed_bytes + dense_bytes + lb_tot * (mixed ? 2 : 8) > budget) return WAVE_TOO_BIG;
     if (!c->lb.ensure(lb_tot * (mixed ? 2 : 8))) return fail(c, QLX_ERR_NOMEM, "Lb pool allocation failed");
     bd.lb = c->lb.p;
     HIPCHK(c, hipMemcpyAsync(c->d_meta.p, meta.data(), sizeof(ItemMeta) * B, hipMemcpyHostToDevice, st));
     timer_begin(c, "lbkernel");
-    if (launch_build_lb_b(st, bd, max_rows, max_nsup, mixed ? 1 : 0, mixed ? 128 : 64) != 0)
+    if (launch_build_lb_b(st, bd, max_rows, mixed ? 1 : 0) != 0)
         return fail(c, QLX_ERR_RANGE, "PSF too large for the Lb build (at most 8192 taps in FP64, 16384 mixed)");
     timer_end(c, "lbkernel");
     timer_end(c, "lbuild");
     // R depends only on the active cells: it is built now and factored (ln det R only) on the second
-    // stream, from a copy, while the main stream forms F (the SYRK, then k_prep_f_b, which reads R
+    // stream, from a copy, while the main stream forms F (the SYRK, then k_add_reg_b, which reads R
     // itself); the streams join before the log-determinants.  (Started before the Lb build instead,
     // its small launches slow that latency-bound kernel by more than they save.)  R's many small
     // launches are enqueued after the SYRK's: the host's time spent enqueueing them then overlaps
@@ -894,19 +894,16 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
         if (!c->Fraw.ensure(f_tot * 8) || !c->d_lam.ensure((size_t)B * 8)) return fail(c, QLX_ERR_NOMEM, "regparam buffers");
         HIPCHK(c, hipMemcpyAsync(c->d_lam.p, lamh.data(), (size_t)B * 8, hipMemcpyHostToDevice, st));
         bd.lam = c->d_lam.as<double>();
+        bd.Fraw = c->Fraw.as<double>();
     }
     launch_curvature_b(st, bd, max_cells, max_rtiles);  // R of the items that hold one
     HIPCHK(c, hipEventRecord(c->ev_fork, st));
     if (!mixed) launch_gather_cvec_b(st, bd, max_rows);
     timer_begin(c, "syrk");
-    if (mixed) launch_syrk_f16_b(st, bd, max_ncb, max_nkt);
-    else launch_syrk_f64_b(st, bd, max_ncb, max_nkt);
+    if (mixed) launch_syrk_f16_b(st, bd, max_ncb);
+    else launch_syrk_f64_b(st, bd, max_ncb);
     timer_end(c, "syrk");
-    if (opt) {
-        HIPCHK(c, hipMemcpyAsync(c->Fraw.p, c->F.p, f_tot * 8, hipMemcpyDeviceToDevice, st));
-        bd.Fraw = c->Fraw.as<double>();
-    }
-    launch_prep_fr_b(st, bd, max_ld, mixed ? 1 : 0);
+    launch_add_reg_b(st, bd, max_ld, max_cells, mixed ? 1 : 0);
     HIPCHK(c, hipStreamWaitEvent(c->stream2, c->ev_fork, 0));
     HIPCHK(c, hipMemcpyAsync(c->Rf.p, c->R.p, r_tot * 8, hipMemcpyDeviceToDevice, c->stream2));
     int max_bwb = 1;
@@ -988,7 +985,7 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
             for (int b = 0; b < B; b++) lamh[b] = meta[b].valid ? pow(10, brent[b].point()) : S.regparam;
             final_pass = all_done;
             HIPCHK(c, hipMemcpyAsync(c->d_lam.p, lamh.data(), (size_t)B * 8, hipMemcpyHostToDevice, st));
-            launch_prep_fr_b(st, bd, max_ld, 0);
+            launch_add_reg_b(st, bd, max_ld, max_cells, 0);
             timer_begin(c, "cholesky");
             {
                 const int rc = factor_on(c, st, c->d_mats.as<MatDesc>(), 0, nF, max_ld / 64, 1, 0, 0);
@@ -1005,10 +1002,10 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
 
     std::vector<double> o((size_t)B * QLX_OUT_STRIDE);
     std::vector<int> stat((size_t)B * 4);
-    std::vector<unsigned long long> nev(B);
+    std::vector<unsigned long long> nev(2 * (size_t)B);
     HIPCHK(c, hipMemcpyAsync(o.data(), bd.out, o.size() * 8, hipMemcpyDeviceToHost, st));
     HIPCHK(c, hipMemcpyAsync(stat.data(), bd.status, stat.size() * 4, hipMemcpyDeviceToHost, st));
-    HIPCHK(c, hipMemcpyAsync(nev.data(), bd.nevals, (size_t)B * 8, hipMemcpyDeviceToHost, st));
+    HIPCHK(c, hipMemcpyAsync(nev.data(), bd.nevals, nev.size() * 8, hipMemcpyDeviceToHost, st));
     HIPCHK(c, hipStreamSynchronize(st));
     timers_collect(c);
     for (int b = 0; b < B; b++) {
@@ -1039,25 +1036,16 @@ int run_wave(Ctx* c, const qlx_lens_model* models, const std::vector<WaveItem>& 
 
     // ---- work accounting over the wave (the launches timed above) ----
     {
-        const std::vector<unsigned>& nzh = c->nzh;  // read back with the support counts
         qlx_stats& T = c->stats;
         memset(&T, 0, sizeof(T));
         for (int b = 0; b < B; b++) {
             const ItemMeta& M = meta[b];
             if (!M.valid) continue;
-            const double cbw = (double)(1 << M.cbs);
-            const double tile = 2.0 * 64 * cbw * cbw;
-            double exec_pairs = 0, nblk = 0;
-            for (int kt = 0; kt < M.nkt; kt++) {
-                double bits = 0;
-                for (int w = 0; w < M.ncbw; w++) bits += __builtin_popcount(nzh[M.nz_off + (size_t)kt * M.ncbw + w]);
-                exec_pairs += bits * (bits + 1) / 2;
-                nblk += bits;
-            }
-            T.syrk_exec_flops += exec_pairs * tile;
-            T.syrk_dense_flops += (double)M.ncb * (M.ncb + 1) / 2 * M.nkt * tile;
+            const double strip = 2.0 * 64 * 16 * 16;  // flops of a pair of 64 x 16 strips
+            T.syrk_exec_flops += (double)nev[B + b] * strip;
+            T.syrk_dense_flops += (double)M.ldN / 16 * (M.ldN / 16 + 1) / 2 * M.nkt * strip;
             T.syrk_alg_flops += (double)M.n_img * M.n_src * (M.n_src + 1) + 2.0 * M.n_img * M.n_src;
-            T.lb_bytes += nblk * 64 * cbw * (mixed ? 2 : 8);
+            T.lb_bytes += (double)M.nblk * 64 * 16 * (mixed ? 2 : 8);
             T.integrand_evals += (double)nev[b];
             T.chol_flops += (double)M.n_src * M.n_src * M.n_src / 3.0;
             T.n_items++;

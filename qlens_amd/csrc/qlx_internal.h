@@ -16,7 +16,6 @@ namespace qlx {
 
 #define QLX_MAX_SRC_AXIS 512
 #define QLX_MAX_LD 16384          // padded source dimension limit of the dense F (n_src <= 16383)
-#define QLX_MAX_CBW 8             // 32-bit support-mask words per 64-row chunk (QLX_MAX_LD / 64 / 32)
 #define QLX_CSC_SEG 512           // row positions per segment of L's column-ordered (CSC) build
 __host__ __device__ inline long long csc_segments(long long s_pix) { return (s_pix + QLX_CSC_SEG - 1) / QLX_CSC_SEG; }
 // per-item source grid block: sxv[513], syv[513], scx[512], scy[512]
@@ -29,7 +28,7 @@ __host__ __device__ inline long long csc_segments(long long s_pix) { return (s_p
                                   // regparam objective (chi^2 over the active pixels + regterms + ln det F), spare
 #define QLX_VEC_SLOTS 8           // per item, ldN doubles each: s (F order), diagF, diagR, Fdiag, resid,
                                   // partial sums, s (reference order), the residual's row-strip sums
-// internal source order: active cells ranked in 8 (x) by 16 (y) cell tiles, tiles y-major
+// internal source order: active cells ranked in 8 (x) by 16 (y) cell tiles of 4 x 4 cells, y-major
 #define QLX_TILE_W 8
 #define QLX_TILE_H 16
 
@@ -67,13 +66,14 @@ __host__ __device__ inline int rays_per_pixel(int nsplit) { return nsplit ? nspl
 struct ItemMeta {
     int valid;                       // item takes part in the dense stages
     int n_src, n_img, ldN, nrows;    // active counts; padded source dim (>= n_src+1); padded rows
-    int ncb, ncbw, nkt;              // column blocks, mask words per chunk, 64-row chunks
-    int snx, sny, bwb, nblk;         // source grid; R band in blocks; Lb support blocks
-    int nsup_max, cbs;               // most support blocks of one chunk; log2 of the Lb column-block width
-    long long lb_off;                // Lb pool (elements: double, or 2 x nblk x 4096 bf16)
+    int ncb, nkt;                    // column blocks of the SYRK, 64-row chunks
+    int nsw, ncw;                    // per chunk: mask words of 16-column strips, of columns
+    int snx, sny, bwb, nblk;         // source grid; R band in blocks; Lb support strips
+    int cbs, pad;                    // log2 of the SYRK's column-block width
+    long long lb_off;                // Lb pool (elements: double or FP16; 64 x 16 a strip)
     long long f_off;                 // F (elements of F or F32)
     long long r_off;                 // banded R tiles (doubles)
-    long long cvec_off, vec_off, nz_off, bb_off, w_off;
+    long long cvec_off, vec_off, nz_off, col_off, sup_off, bb_off, w_off;
     long long keep_off;              // byte offset of the item's solution block in the keep buffer
 };
 
@@ -90,7 +90,7 @@ struct BatchDev {
     int pnx, pny;
     double tol, lambda;
     const double* lam;          // per-item lambda (regparam optimisation), or null: lambda for every item
-    const double* Fraw;         // FP64 F as the SYRK formed it (regparam optimisation), or null
+    double* Fraw;               // where the SYRK forms FP64 F when it is kept (regparam optimisation), or null
     // per-item inputs
     const ModelPrep* models;
     const double* sgrid;        // QLX_SG_STRIDE doubles per item
@@ -110,7 +110,7 @@ struct BatchDev {
     int* rrep;                  // 1 per item: the first item of the wave with the same R (itself if none)
     int* pidx;                  // s_pix
     int* act_pix;               // s_pix
-    int* counts;                // 4 per item: n_src, n_img, support blocks, largest chunk support
+    int* counts;                // 4 per item: n_src, n_img, support strips, spare
     int* ucol;                  // s_pix*3*nsub
     double* uval;               // s_pix*3*nsub
     int* ucnt;                  // s_pix
@@ -120,8 +120,6 @@ struct BatchDev {
                                 // the entries per L column, then the segment's first slot in it
     unsigned* cpix;             // s_pix*3*nsub: L by columns, ordered: pixel (i << 16 | j) of each entry
     double* cval;               // s_pix*3*nsub: L by columns, ordered: value of each entry
-    unsigned* pmask;            // s_pix*QLX_MAX_CBW: column blocks touched by each active pixel's L row
-    unsigned* hmask;            // s_pix*QLX_MAX_CBW per grid pixel (y-major): pmask ORed over the PSF's x window
     double s16;                 // mixed path: power of two that scales the FP16 pool entries (|x s16| <= 2^14)
     int* key;                   // s_pix: row-order position of each active row
     int* bcnt;                  // s_cell+2: entries per L column
@@ -129,6 +127,7 @@ struct BatchDev {
     int* bfill;                 // s_cell+2: scatter cursors
     int* perm;                  // s_pix: active row at each row-order position
     unsigned long long* nevals; // 1 per item
+    unsigned long long* npairs; // 1 per item: pairs of strips of one chunk
     long long s_pix, s_cell;
     // pools and outputs
     const ItemMeta* meta;
@@ -142,8 +141,10 @@ struct BatchDev {
     double* vec;                // QLX_VEC_SLOTS * ldN doubles per item
     double* zres;               // mixed: the refinement residual's transposed tile products, ldN^2 / 128
                                 // doubles per item (at f_off / 128)
-    unsigned* nz;               // nkt * ncbw support words per item
-    int* bbase;                 // nkt + 1 slot bases per item
+    unsigned* nz;               // nkt * nsw support words per item: the 16-column strips a chunk holds
+    unsigned* colb;             // nkt * ncw words per item: the columns with an entry in a chunk's reach
+    unsigned* sup;              // ncb * nkt per item: a chunk's strips in a column block (k_sup_table_b)
+    int* bbase;                 // nkt + 1 slot bases (strips) per item
     double* winv;               // per item 2 * ldN*64 doubles (F then R block inverses)
     double* model;              // per item 2*s_pix
     double* out;                // QLX_OUT_STRIDE per item
@@ -247,18 +248,19 @@ void launch_compact_b(hipStream_t s, const BatchDev& bd);
 void launch_merge_lrows_b(hipStream_t s, const BatchDev& bd, int max_img);
 void launch_sort_rows_b(hipStream_t s, const BatchDev& bd, int max_img, int max_src);
 void launch_lcols_b(hipStream_t s, const BatchDev& bd, int max_img, int max_src);
-void launch_row_support_b(hipStream_t s, const BatchDev& bd, int max_nkt);
-int launch_build_lb_b(hipStream_t s, const BatchDev& bd, int max_rows, int max_nsup, int mixed, int cbw);
+void launch_row_support_b(hipStream_t s, const BatchDev& bd, int max_nkt, int max_ld, int max_sup);
+int launch_build_lb_b(hipStream_t s, const BatchDev& bd, int max_rows, int mixed);
 void launch_gather_cvec_b(hipStream_t s, const BatchDev& bd, int max_rows);
-void launch_syrk_f64_b(hipStream_t s, const BatchDev& bd, int max_ncb, int max_nkt);
-void launch_syrk_f16_b(hipStream_t s, const BatchDev& bd, int max_ncb, int max_nkt);
+void launch_syrk_f64_b(hipStream_t s, const BatchDev& bd, int max_ncb);
+void launch_syrk_f16_b(hipStream_t s, const BatchDev& bd, int max_ncb);
 void launch_curvature_b(hipStream_t s, const BatchDev& bd, int max_cells, int max_rtiles);
 // items whose R equals an earlier item's (same grid shape and active-index map) get rrep = that item,
 // others rrep = themselves: one build and one factorization of R serve them all (the host reads rrep
 // back and gives R's factorization the representatives' descriptors only; launch_curvature_b
 // builds the representatives' R only)
 void launch_rdup_b(hipStream_t s, const BatchDev& bd);
-void launch_prep_fr_b(hipStream_t s, const BatchDev& bd, int max_ld, int f32);
+// F += lambda R (FP64: F copied from Fraw first, when F as formed is kept there)
+void launch_add_reg_b(hipStream_t s, const BatchDev& bd, int max_ld, int max_cells, int f32);
 // panel_blocks: width of the FP32 dense schedule's panels in 64-blocks (a multiple of 4; 0 = 16);
 // the factor is bitwise the same for every width
 void cholesky_batched(hipStream_t s, const MatDesc* d_mats, int n32, int n64, int max_nb, int dense, int max_bwb,

@@ -1,0 +1,66 @@
+"""The blurred-L pool's strips and the SYRK over them, at the sizes where strips, column blocks, chunks
+and the tap table end: chunks that span two ends of an image row (thin masks and images), PSFs of one pixel
+to wider than the padded tap table takes, source grids whose last strip, block and data column fall at
+every place, and more chunks than one list holds; against the oracle, FP64 and mixed."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from qlens_amd import qlx
+from qlens_amd import workloads as W
+
+TOL = 1e-9         # FP64: the oracle's sums in another order
+TOL_MIXED = 0.1    # |delta ln E| of the mixed path's contract
+
+
+def _psf(n, m):
+    x, y = np.arange(n) - n // 2, np.arange(m) - m // 2
+    p = np.exp(-0.5 * ((x[:, None] / (0.25 * n)) ** 2 + (y[None, :] / (0.25 * m)) ** 2))
+    return p / p.sum()
+
+
+def _thin(nx, ny):
+    m = np.zeros((nx, ny), np.uint8)
+    m[::3] = 1       # every third column of pixels: chunks of many image tiles
+    m[:, :5] = 1
+    m[:, -4:] = 1
+    return m
+
+
+CASES = [
+    # nx, ny, nsplit, source grid, psf, mask
+    (40, 44, 2, (15, 1 + 16), (1, 1), None),
+    (40, 44, 2, (8, 16), (3, 5), "thin"),
+    (61, 37, 1, (12, 10), (9, 3), "thin"),
+    (50, 50, 2, (23, 23), (61, 61), None),   # no padded tap table in FP64
+    (60, 50, 2, (16, 16), (65, 65), None),   # none in either precision
+    (36, 220, 0, (31, 9), (5, 5), None),
+    (200, 190, 0, (17, 13), (3, 3), None),   # over 512 chunks: more than one list
+]
+
+
+def _case(nx, ny, nsplit, src_n, psf, mask):
+    xv, yv = W.corners(-2.2, 2.2, nx), W.corners(-2.0, 2.0, ny)
+    base = W.c1()
+    return dict(name="strips", xvals=xv, yvals=yv, nsplit=nsplit, lenses=base["lenses"], sources=base["sources"],
+                psf=_psf(*psf), sigma=0.02, seed=3, srcgrid=(-2.4, 2.4, -2.3, 2.3), src_n=src_n, regparam=50.0, integral_tol=1e-6,
+                mask=_thin(nx, ny) if mask else None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("args", CASES)
+@pytest.mark.parametrize("precision", [qlx.QLX_PREC_FP64, qlx.QLX_PREC_MIXED])
+def test_strips_match_oracle(qlx_ctx, args, precision):
+    case = _case(*args)
+    data = O.mock_image(case)
+    ref, arr = O.invert(case, data)
+    qlx_ctx.load_workload(case, data, precision=precision)
+    r = qlx_ctx.invert_image_surface_brightness_map(case["lenses"])[0]
+    assert r["status"] == 0 and (r["n_src_active"], r["n_img_active"]) == (ref["n_src"], ref["n_img"])
+    if precision == qlx.QLX_PREC_MIXED:
+        assert abs(r["minus2lnE"] - ref["minus2lnE"]) / 2 < TOL_MIXED
+        return
+    for k in ("minus2lnE", "chisq0", "logdetF", "logdetR"):
+        assert abs(r[k] - ref[k]) <= TOL * max(1.0, abs(ref[k])), k
+    src = qlx_ctx.get_source()["src"]
+    assert np.linalg.norm(src - arr["src"]) <= TOL * np.linalg.norm(arr["src"])
