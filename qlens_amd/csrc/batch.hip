@@ -2552,7 +2552,7 @@ __device__ __forceinline__ void chol_diag_f64_lds(const MatDesc& D, int kb, doub
 // next one, so a column needs this one launch instead of a diagonal, a panel and a panel-update one.
 // Alone, a step is bound by that workgroup's serial chain (its 64^3 products at 1.7 us each on one CU,
 // then the diagonal block); the grid is (matrices, row blocks), so it is dispatched first.
-// One 3712 matrix alone: 4.3 -> 2.15 ms for the factorization, R's banded chain of 58 steps 3.0 -> 1.3.
+// One 3712 matrix alone: 4.3 -> 2.15 ms for the factorization, R's banded chain of 58 steps 3.0 -> 1.6.
 __global__ void __launch_bounds__(256) k_chol_lpanel_f64(const MatDesc* mats, int kb, int k0, int kend)
 {
     __shared__ __attribute__((aligned(16))) double sm[DGL];  // stages, operand tiles, the diagonal block's buffers
@@ -2911,35 +2911,228 @@ __device__ void tri_bwd(const T* L, int ld, int nb, const T* W, T* sx, T (*part)
     }
 }
 
+// Solves by panels of 256 rows: the panel's triangle (block by block, tri_bwd / tri_fwd), then its products
+// off every panel still to be solved.  Two forms of the same arithmetic, so the same bits:
+//   * a launch per panel (k_solve_bwd_b, k_solve_fwd_b), each panel still to be solved a workgroup, so
+//     that an item's factor is read by many CUs: workgroup g of step s takes panel P -/+ g, subtracts
+//     the products of the panel solved by the launch before, and workgroup 0 solves P's triangle;
+//   * one workgroup per item for the whole solve (k_solve_one_b), where the items fill the GPU by
+//     themselves and the launches' tails would only idle it.
+// A solve reads its factor once; one workgroup gets the 55-110 GB/s of its CU, a launch per panel costs a
+// chain of a triangle and a product (~20 us) each.  The stage, one workgroup -> launches: 6 items of 10 000
+// mixed 12.2 -> 3.2 ms, one of 3712 mixed 1.21 -> 0.65, FP64 0.62 -> 0.31; one -> launches: 256 items of
+// 3712 mixed 6.6 -> 7.9 ms, 100 FP64 1.34 -> 1.42, so these keep the one workgroup.  The vector stands in slot 6 of the item's vectors, in the factor's type.
+#define PAN 256
+#define SOLVE_ONE_B 96      // items from which one workgroup each is the better form,
+#define SOLVE_ONE_LD 8192   // for factors whose vector fits LDS beside the partial sums (107 KB of FP64)
+#define SOLVE_ONE_LDS(ld) (16 * PAN + 16 * (TS + 1) + TS + (size_t)(ld))
 template <typename T>
-__global__ void __launch_bounds__(1024) k_trisolve_b(BatchDev bd)
+__device__ __forceinline__ T* solve_vec(const BatchDev& bd, const ItemMeta& M) { return (T*)(bd.vec + M.vec_off + 6 * (size_t)M.ldN); }
+
+// part[w][c]: wave w's sum over its rows (w, w + 16, ..) of the panel's L(r, c) x(r); Lp = the panel's
+// first row at the target panel's first column, nr rows (a multiple of 128), x their values
+template <typename T>
+__device__ __forceinline__ void bwd_tile(const T* Lp, int ld, int nr, const T* x, T (*part)[PAN])
 {
-    extern __shared__ double sx_raw[];
-    __shared__ T part[16][TS + 1];
+    constexpr int VW = 16 / sizeof(T);
+    typedef T P __attribute__((ext_vector_type(VW)));
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int h = 0; h < PAN; h += 64 * VW) {
+        const T* Lw = Lp + (size_t)w * ld + h + VW * lane;
+        P acc = (P)0;
+#pragma unroll 1
+        for (int k0 = 0; 16 * k0 < nr; k0 += 8) {  // eight rows in flight
+            P t[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) t[k] = *(const P*)(Lw + (size_t)(16 * (k0 + k)) * ld);
+#pragma unroll
+            for (int k = 0; k < 8; k++) acc = __builtin_elementwise_fma(t[k], (P)x[w + 16 * (k0 + k)], acc);
+        }
+        *(P*)&part[w][h + VW * lane] = acc;
+    }
+}
+template <typename T>
+__device__ __forceinline__ T part_sum(const T (*part)[PAN], int c)
+{
+    T t = part[0][c];
+#pragma unroll
+    for (int w = 1; w < 16; w++) t += part[w][c];
+    return t;
+}
+
+// row w + 16 (lane >> 2) of the target panel (nq rows, a multiple of 128): its sum of L(r, c) x(c) over the
+// 256 columns of a solved panel (all four lanes of a row); Lp = its first row at that panel's first column
+__device__ __forceinline__ float fwd_tile(const float* Lp, int ld, int nq, const float* x)
+{
+    typedef float T;
+    typedef float4_t P;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const P xc = *(const P*)(x + 4 * lane);
+    const T* Lw = Lp + (size_t)w * ld + 4 * lane;
+    T a[16];
+#pragma unroll
+    for (int k0 = 0; k0 < 16; k0 += 8) {
+        P t[8];
+        if (16 * k0 < nq)
+#pragma unroll
+            for (int k = 0; k < 8; k++) t[k] = *(const P*)(Lw + (size_t)(16 * (k0 + k)) * ld);
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const P m = t[k] * xc;
+            a[k0 + k] = 16 * k0 < nq ? (m.x + m.y) + (m.z + m.w) : 0;
+        }
+    }
+    // 16 row sums over 64 lanes: four halvings, then a 4-lane sum
+    T b[8], c[4], d[2];
+    const bool h5 = lane & 32, h4 = lane & 16, h3 = lane & 8, h2 = lane & 4;
+#pragma unroll
+    for (int j = 0; j < 8; j++) b[j] = (h5 ? a[8 + j] : a[j]) + __shfl_xor(h5 ? a[j] : a[8 + j], 32, 64);
+#pragma unroll
+    for (int j = 0; j < 4; j++) c[j] = (h4 ? b[4 + j] : b[j]) + __shfl_xor(h4 ? b[j] : b[4 + j], 16, 64);
+#pragma unroll
+    for (int j = 0; j < 2; j++) d[j] = (h3 ? c[2 + j] : c[j]) + __shfl_xor(h3 ? c[j] : c[2 + j], 8, 64);
+    T e = (h2 ? d[1] : d[0]) + __shfl_xor(h2 ? d[0] : d[1], 4, 64);
+    e += __shfl_xor(e, 2, 64);
+    return e + __shfl_xor(e, 1, 64);
+}
+
+// mode 0: x = L^-T y, y = row n of the factor, to s.  mode 1: y = the vector (of items not yet
+// converged), s += x
+template <typename T>
+__global__ void __launch_bounds__(1024) k_solve_bwd_b(BatchDev bd, int s, int mode)
+{
+    __shared__ T part[16][PAN];
+    __shared__ __align__(16) T sx[PAN];
+    __shared__ T tpart[16][TS + 1];
     __shared__ T rhs[TS];
-    T* sx = (T*)sx_raw;
     const int item = blockIdx.y;
     const ItemMeta& M = bd.meta[item];
-    if (!M.valid) return;
-    const int ld = M.ldN, nb = ld / TS, n = M.n_src;
+    if (!M.valid || (mode && bd.status[4 * item + 3])) return;
+    const int ld = M.ldN, n = M.n_src, np = (ld + PAN - 1) / PAN;
+    const int Pn = np - 1 - s, Q = Pn - (int)blockIdx.x;  // an item's steps count from its own last panel
+    if (Q < 0) return;
+    const T* L = (sizeof(T) == 8) ? (const T*)(bd.F + M.f_off) : (const T*)(bd.F32 + M.f_off);
+    T* v = solve_vec<T>(bd, M);
+    const int q0 = Q * PAN, nq = min(PAN, ld - q0), c = threadIdx.x;
+    if (s > 0) {
+        const int r0 = (Pn + 1) * PAN;
+        bwd_tile<T>(L + (size_t)r0 * ld + q0, ld, min(PAN, ld - r0), v + r0, part);
+        __syncthreads();
+    }
+    if (c < nq) {
+        // mode 0: until its first update a panel's y stands in row n of the factor
+        T a = (mode || s > 1) ? v[q0 + c] : q0 + c < n ? L[(size_t)n * ld + q0 + c] : (T)0;
+        if (s > 0) a -= part_sum<T>(part, c);
+        sx[c] = a;
+    }
+    __syncthreads();
+    if (blockIdx.x == 0) {
+        tri_bwd<T>(L + (size_t)q0 * ld + q0, ld, nq / TS, (const T*)(bd.winv + M.w_off) + (size_t)q0 * TS, sx, tpart, rhs);
+        double* so = bd.vec + M.vec_off + q0;
+        if (c < nq) {
+            if (mode == 0) so[c] = q0 + c < n ? (double)sx[c] : 0.0;
+            else if (q0 + c < n) so[c] += (double)sx[c];
+        }
+    }
+    if (c < nq) v[q0 + c] = sx[c];
+}
+
+// x = L^-1 b in place in the vector, of items not yet converged (FP32)
+__global__ void __launch_bounds__(1024) k_solve_fwd_b(BatchDev bd, int s)
+{
+    __shared__ __align__(16) float sx[PAN];
+    __shared__ float tpart[16][TS + 1];
+    __shared__ float rhs[TS];
+    const int item = blockIdx.y;
+    const ItemMeta& M = bd.meta[item];
+    if (!M.valid || bd.status[4 * item + 3]) return;
+    const int ld = M.ldN, np = (ld + PAN - 1) / PAN;
+    const int Q = s + (int)blockIdx.x;
+    if (Q >= np) return;
+    const float* L = bd.F32 + M.f_off;
+    float* v = solve_vec<float>(bd, M);
+    const int q0 = Q * PAN, nq = min(PAN, ld - q0), c = threadIdx.x;
+    const int r = (c >> 6) + 16 * ((c & 63) >> 2);
+    if (s > 0) {
+        const int c0 = (s - 1) * PAN;
+        const float e = fwd_tile(L + (size_t)q0 * ld + c0, ld, nq, v + c0);
+        if ((c & 3) == 0 && r < nq) sx[r] = v[q0 + r] - e;
+    } else if (c < nq) {
+        sx[c] = v[q0 + c];
+    }
+    __syncthreads();
+    if (blockIdx.x == 0) tri_fwd<float>(L + (size_t)q0 * ld + q0, ld, nq / TS, (const float*)(bd.winv + M.w_off) + (size_t)q0 * TS, sx, tpart, rhs);
+    if (c < nq) v[q0 + c] = sx[c];
+}
+
+// mode 0: x = L^-T y to s.  mode 1 (FP32): s += (L L^T)^-1 of the vector, of items not yet converged
+template <typename T>
+__global__ void __launch_bounds__(1024) k_solve_one_b(BatchDev bd, int mode)
+{
+    extern __shared__ __align__(16) double one_lds[];
+    T(*part)[PAN] = (T(*)[PAN])one_lds;
+    T(*tpart)[TS + 1] = (T(*)[TS + 1])(part + 16);
+    T* rhs = (T*)(tpart + 16);
+    T* sx = rhs + TS;  // the vector
+    const int item = blockIdx.y;
+    const ItemMeta& M = bd.meta[item];
+    if (!M.valid || (mode && bd.status[4 * item + 3])) return;
+    const int ld = M.ldN, n = M.n_src, np = (ld + PAN - 1) / PAN, tid = threadIdx.x;
     const T* L = (sizeof(T) == 8) ? (const T*)(bd.F + M.f_off) : (const T*)(bd.F32 + M.f_off);
     const T* W = (const T*)(bd.winv + M.w_off);
-    for (int c = threadIdx.x; c < ld; c += 1024) sx[c] = (c < n) ? L[(size_t)n * ld + c] : (T)0;
+    const T* v = solve_vec<T>(bd, M);
+    for (int c = tid; c < ld; c += 1024) sx[c] = mode ? v[c] : c < n ? L[(size_t)n * ld + c] : (T)0;
     __syncthreads();
-    tri_bwd<T>(L, ld, nb, W, sx, part, rhs);
+    if constexpr (sizeof(T) == 4)
+        if (mode)
+            for (int P = 0; P < np; P++) {
+                const int p0 = P * PAN;
+                tri_fwd<T>(L + (size_t)p0 * ld + p0, ld, min(PAN, ld - p0) / TS, W + (size_t)p0 * TS, sx + p0, tpart, rhs);
+                const int r = (tid >> 6) + 16 * ((tid & 63) >> 2);
+                for (int q0 = p0 + PAN; q0 < ld; q0 += PAN) {
+                    const int nq = min(PAN, ld - q0);
+                    const float e = fwd_tile(L + (size_t)q0 * ld + p0, ld, nq, sx + p0);
+                    if ((tid & 3) == 0 && r < nq) sx[q0 + r] -= e;
+                }
+                __syncthreads();
+            }
+    for (int P = np - 1; P >= 0; P--) {
+        const int p0 = P * PAN, npr = min(PAN, ld - p0);
+        tri_bwd<T>(L + (size_t)p0 * ld + p0, ld, npr / TS, W + (size_t)p0 * TS, sx + p0, tpart, rhs);
+        for (int Q = P - 1; Q >= 0; Q--) {
+            bwd_tile<T>(L + (size_t)p0 * ld + Q * PAN, ld, npr, sx + p0, part);
+            __syncthreads();
+            if (tid < PAN) sx[Q * PAN + tid] -= part_sum<T>(part, tid);
+            __syncthreads();
+        }
+    }
     double* s = bd.vec + M.vec_off;
-    for (int c = threadIdx.x; c < ld; c += 1024) s[c] = (c < n) ? (double)sx[c] : 0.0;
+    for (int c = tid; c < ld; c += 1024) {
+        if (mode == 0) s[c] = (c < n) ? (double)sx[c] : 0.0;
+        else if (c < n) s[c] += (double)sx[c];
+    }
+}
+
+template <typename T>
+static void launch_solve(hipStream_t s, const BatchDev& bd, int max_ld, int mode, bool one)
+{
+    const int np = (max_ld + PAN - 1) / PAN;
+    if (one && max_ld <= SOLVE_ONE_LD) {
+        allow_big_lds((const void*)k_solve_one_b<T>);
+        hipLaunchKernelGGL(k_solve_one_b<T>, dim3(1, bd.B), dim3(1024), SOLVE_ONE_LDS(max_ld) * sizeof(T), s, bd, mode);
+        return;
+    }
+    if (mode)
+        for (int k = 0; k < np; k++) hipLaunchKernelGGL(k_solve_fwd_b, dim3(np - k, bd.B), dim3(1024), 0, s, bd, k);
+    for (int k = 0; k < np; k++) hipLaunchKernelGGL(k_solve_bwd_b<T>, dim3(np - k, bd.B), dim3(1024), 0, s, bd, k, mode);
 }
 
 void launch_trisolve_b(hipStream_t s, const BatchDev& bd, int max_ld, int f32)
 {
-    if (f32) {
-        allow_big_lds((const void*)k_trisolve_b<float>);
-        hipLaunchKernelGGL(k_trisolve_b<float>, dim3(1, bd.B), dim3(1024), (size_t)max_ld * 4, s, bd);
-    } else {
-        allow_big_lds((const void*)k_trisolve_b<double>);
-        hipLaunchKernelGGL(k_trisolve_b<double>, dim3(1, bd.B), dim3(1024), (size_t)max_ld * 8, s, bd);
-    }
+    const bool one = bd.B >= SOLVE_ONE_B;
+    if (f32) launch_solve<float>(s, bd, max_ld, 0, one);
+    else launch_solve<double>(s, bd, max_ld, 0, one);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -3110,24 +3303,17 @@ __global__ void __launch_bounds__(64) k_resid_cols_b(BatchDev bd)
     }
 }
 
-// one refinement step per item: check convergence from the residual partials, else correct s
-__global__ void __launch_bounds__(1024) k_refine_b(BatchDev bd, int final_check, double tol)
+// convergence of the item from the residual partials; an item that goes on gets the residual into its vector
+__global__ void __launch_bounds__(1024) k_refine_check_b(BatchDev bd, int final_check, double tol)
 {
-    extern __shared__ double sx_raw[];
-    __shared__ float part[16][TS + 1];
-    __shared__ float rhs[TS];
     __shared__ double red[2][64];
     __shared__ int done;
-    float* sx = (float*)sx_raw;
     const int item = blockIdx.y;
     const ItemMeta& M = bd.meta[item];
     if (!M.valid || bd.status[4 * item + 3]) return;
     const int ld = M.ldN, nb = ld / TS, n = M.n_src;
     const int tid = threadIdx.x;
-    double* v = bd.vec + M.vec_off;
-    double* s = v;
-    const double* r = v + 4 * (size_t)ld;
-    const double* pr = v + 5 * (size_t)ld;
+    const double* pr = bd.vec + M.vec_off + 5 * (size_t)ld;
     const int nbr = (n + TS - 1) / TS;
     if (tid < 64) {
         double a = 0.0, b = 0.0;
@@ -3153,23 +3339,20 @@ __global__ void __launch_bounds__(1024) k_refine_b(BatchDev bd, int final_check,
     }
     __syncthreads();
     if (done) return;
-    const float* L = bd.F32 + M.f_off;
-    const float* W = (const float*)(bd.winv + M.w_off);
-    for (int c = tid; c < ld; c += 1024) sx[c] = (c < n) ? (float)r[c] : 0.0f;
-    __syncthreads();
-    tri_fwd<float>(L, ld, nb, W, sx, part, rhs);
-    tri_bwd<float>(L, ld, nb, W, sx, part, rhs);
-    for (int c = tid; c < n; c += 1024) s[c] += (double)sx[c];
+    float* v = solve_vec<float>(bd, M);
+    const double* r = bd.vec + M.vec_off + 4 * (size_t)ld;
+    for (int c = tid; c < ld; c += 1024) v[c] = (c < n) ? (float)r[c] : 0.0f;
 }
 
 void launch_refine_b(hipStream_t s, const BatchDev& bd, int max_ld, int iters, double tol)
 {
     const int nb = max_ld / TS;
-    allow_big_lds((const void*)k_refine_b);
     for (int it = 0; it <= iters; it++) {
         hipLaunchKernelGGL(k_resid_rows_b, dim3(nb, bd.B), dim3(256), 0, s, bd);
         hipLaunchKernelGGL(k_resid_cols_b, dim3(nb, bd.B), dim3(64), 0, s, bd);
-        hipLaunchKernelGGL(k_refine_b, dim3(1, bd.B), dim3(1024), (size_t)max_ld * 4, s, bd, it == iters ? 1 : 0, tol);
+        hipLaunchKernelGGL(k_refine_check_b, dim3(1, bd.B), dim3(1024), 0, s, bd, it == iters ? 1 : 0, tol);
+        // steps after the first are for the few items still above the tolerance: one launch each
+        if (it < iters) launch_solve<float>(s, bd, max_ld, 1, it > 0 || bd.B >= SOLVE_ONE_B);
     }
 }
 

@@ -1,0 +1,34 @@
+"""The triangular solves by panels of 256 rows, at the sizes where panels end (one panel, an edge, a
+remainder, several): a launch per panel (few items) against the oracle, and against one workgroup per item
+(many items), which does the same arithmetic and so has to give the same bits; FP64, and FP32 with its
+refinement."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from qlens_amd import qlx
+from qlens_amd import workloads as W
+
+TOL = 1e-9          # FP64: the oracle's sums in another order
+TOL_MIXED = 1e-4    # mixed: refined to an FP64 residual of 1e-10 of the right side, on systems of condition below 1e6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("src_n", [(5, 4), (14, 9), (16, 16), (17, 15), (20, 18), (26, 24), (30, 29)])
+@pytest.mark.parametrize("precision", [qlx.QLX_PREC_FP64, qlx.QLX_PREC_MIXED])
+def test_panel_solves(qlx_ctx, src_n, precision):
+    case = W.c1()
+    case["src_n"] = src_n
+    data = O.mock_image(case)
+    _, arr = O.invert(case, data)
+    qlx_ctx.load_workload(case, data, precision=precision)
+    models = [case["lenses"]] + W.proposals(case, 99, 3)
+    one = qlx_ctx.invert_image_surface_brightness_map(models[0])[0]
+    src1 = qlx_ctx.get_source()["src"]
+    tol = TOL_MIXED if precision == qlx.QLX_PREC_MIXED else TOL
+    assert one["status"] == 0
+    assert np.linalg.norm(src1 - arr["src"]) <= tol * np.linalg.norm(arr["src"])
+    many = qlx_ctx.invert_image_surface_brightness_map(models)
+    for k in ("minus2lnE", "chisq0", "Es"):
+        assert one[k] == many[0][k], k
+    assert np.array_equal(qlx_ctx.get_source(0)["src"], src1)
