@@ -206,7 +206,7 @@ def main():
                  "syrk_f64_executed_tflops": round(ps["syrk_exec_flops"] / syrk_s / 1e12, 2) if syrk_s else None,
                  "syrk_f64_executed_frac_of_fp64_peak": round(ps["syrk_exec_flops"] / syrk_s / 1e12 / PEAK_FP64_TFLOPS, 4)
                  if syrk_s else None,
-                 "note": "executed = MFMA flops of the nonzero 64x64 blocks; the dense-equivalent count "
+                 "note": "executed = MFMA flops of the pairs of 64x16 strips; the dense-equivalent count "
                          "N_img*N_src*(N_src+1) is not a rate of this kernel"}
 
     # fast path: mixed precision, B proposals per call.  FP64 ray shooting: the FP32 quadrature
@@ -283,8 +283,8 @@ def main():
     # rooflines, per launch (= one wave of B items), from HIP-event times on the library's stream.
     # Lb build: the largest kernel; HBM-bound by algorithm: it writes the FP16 pool of blurred rows
     # (bytes counted from the support masks) and reads only the CSR L rows (under 3 % of that).
-    # SYRK: block-sparse MFMA work, 2 * 64 * 128^2 flops per pair of nonzero 64 x 128 pool blocks of
-    # one row chunk (the dense-equivalent count would exceed the peak and is not a rate).
+    # SYRK: block-sparse MFMA work, 2 * 64 * 16^2 flops per pair of 64 x 16 pool strips of one row
+    # chunk (the dense-equivalent count would exceed the peak and is not a rate).
     lb_s, syrk_s, ray_s = mean_s(kt["lbkernel"]), mean_s(kt["syrk"]), mean_s(kt["raytrace"])
     roof, roof_syrk, roof_ray = None, None, None
     # ray shooting: VALU-bound; algorithmic flops = counted integrand evaluations x C_INT, the
@@ -308,7 +308,7 @@ def main():
         roof_syrk = {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_F16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_F16_TFLOPS, 4), "traffic": read_traffic("syrk_f16_c2_traffic"),
                      "kernel": "k_syrk_f16_b (F = Lb^T C Lb: FP16 pool, FP32 accumulation, 128x128 tiles over "
-                               "nonzero blocks)",
+                               "the strips a chunk's rows reach)",
                      "items_per_launch": st["n_items"], "flops_block_sparse_per_launch": st["syrk_exec_flops"],
                      "pool_bytes_per_launch": st["lb_bytes"], "avg_launch_ms": round(syrk_s * 1e3, 3)}
 
