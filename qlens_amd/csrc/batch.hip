@@ -2759,7 +2759,7 @@ void launch_logdets_b(hipStream_t s, const BatchDev& bd, int f32)
 }
 
 // ------------------------------------------------------------------------------------------------
-// Triangular solves with the stored block inverses (one workgroup per item).
+// Triangular solves with the stored block inverses.
 // y = L^-1 D is row n of the augmented factor, so the first solve is backward only: x = L^-T y.
 // ------------------------------------------------------------------------------------------------
 // Each block step: a strip product over the solved part of the vector (16 B loads, eight in flight

@@ -27,7 +27,8 @@ __host__ __device__ inline long long csc_segments(long long s_pix) { return (s_p
 #define QLX_OUT_STRIDE 10         // -2lnE, chisq, logdetF, logdetR, Es, regterms, refine_resid, refine_steps,
                                   // regparam objective (chi^2 over the active pixels + regterms + ln det F), spare
 #define QLX_VEC_SLOTS 8           // per item, ldN doubles each: s (F order), diagF, diagR, Fdiag, resid,
-                                  // partial sums, s (reference order), the residual's row-strip sums
+                                  // partial sums, the solves' vector and then s (reference order),
+                                  // the residual's row-strip sums
 // internal source order: active cells ranked in 8 (x) by 16 (y) cell tiles of 4 x 4 cells, y-major
 #define QLX_TILE_W 8
 #define QLX_TILE_H 16
