@@ -2133,7 +2133,7 @@ __device__ __forceinline__ void z_steps(double (&x)[4], const double (&mc)[15], 
 //     (A = M P M^T, M unit lower): a column's chain is its pivot's reciprocal, one product and the next
 //     pivot's update, with the next two columns' entries broadcast by readlane; the other columns take
 //     theirs from LDS a column later, and the sixteen 1 / sqrt(p) are formed at once afterwards;
-//   * the waves after t then update their panels' blocks with v_mfma_f64_16x16x4f64 (operands M P and
+//   * the waves after t then update their panels' blocks with v_mfma_f64_16x16x4f64 (operands M |P| and
 //     M), held in the accumulator layout until their turn;
 //   * wave j owns column block j of M^-1: Z_jj by eliminating the identity while wave j + 1 factors,
 //     then Z_ij = -Z_ii sum_k M_ik Z_kj on MFMA as the Z_ii appear (an accumulator is a B operand as it
@@ -2163,7 +2163,7 @@ __device__ __forceinline__ void chol_diag_f64_4w(const MatDesc& D, int kb, doubl
         for (int s = 0; s < 4; s++) {
             const int c = 16 * t + 4 * s + g;
             b[s] = Mt[c][w16 + m];
-            const T pc = -Pv[c];
+            const T pc = -fabs(Pv[c]);  // L L^T with sqrt|p|, as within the panel
 #pragma unroll
             for (int i = i0; i < 4; i++) av[s][i] = Mt[c][16 * i + m] * pc;
         }

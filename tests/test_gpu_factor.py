@@ -46,3 +46,21 @@ def test_wide_panels_give_the_bits_of_narrow_ones(qlx_ctx):
         one = qlx_ctx.invert_image_surface_brightness_map(models[b])[0]
         for k in ("minus2lnE", "logdetF", "logdetR", "Es"):
             assert one[k] == many[b][k], (b, k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("src_n,lam", [((4, 5), -3e4), ((4, 12), -3e3), ((4, 12), -1e4), ((4, 20), -300.0)])
+def test_negative_pivots_continue_with_their_magnitude(qlx_ctx, src_n, lam):
+    """An indefinite F: the item fails, and its factorization goes on with sqrt|p| in every column
+    (pixelgrid.cpp:17071-17105), across the 16-column panels of a diagonal block and its blocks.  At four
+    cells a row F's column order is the oracle's, so ln det F is comparable.  A relative change of 1e-13 in
+    lambda moves the oracle's by at most 2.1e-5 in these cases (the growth behind a negative pivot), and
+    another order of the sums is a smaller change."""
+    case = _case(src_n)
+    case["regparam"] = lam
+    data = O.mock_image(case)
+    ref, _ = O.invert(case, data, want_arrays=False)
+    qlx_ctx.load_workload(case, data)
+    r = qlx_ctx.invert_image_surface_brightness_map(case["lenses"])[0]
+    assert qlx.STATUS[r["status"]] == "not positive definite" and r["n_src_active"] == ref["n_src"]
+    assert abs(r["logdetF"] - ref["logdetF"]) <= 1e-4
