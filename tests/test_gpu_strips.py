@@ -64,3 +64,21 @@ def test_strips_match_oracle(qlx_ctx, args, precision):
         assert abs(r[k] - ref[k]) <= TOL * max(1.0, abs(ref[k])), k
     src = qlx_ctx.get_source()["src"]
     assert np.linalg.norm(src - arr["src"]) <= TOL * np.linalg.norm(arr["src"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("thin,psf,precision", [(False, 121, qlx.QLX_PREC_MIXED), (True, 121, qlx.QLX_PREC_MIXED), (True, 89, qlx.QLX_PREC_FP64)])
+def test_chunk_support_costs_less_than_the_pool(qlx_ctx, thin, psf, precision):
+    """Finding the columns that a chunk reaches looks at each pixel of its reach once; the pool's build
+    multiplies each of that pixel's entries for 64 rows.  So the stage ahead of the build (L's rows and
+    columns, the supports) takes less time than the build also where large PSFs meet chunks of many image
+    tiles."""
+    case = _case(200, 200, 2, (60, 60), (psf, psf), "thin" if thin else None)
+    case["srcgrid"] = (-0.7, 0.7, -0.7, 0.7)
+    qlx_ctx.load_workload(case, np.ones((200, 200)), precision=precision)
+    ahead, build = [], []
+    for _ in range(6):
+        assert qlx_ctx.invert_image_surface_brightness_map(case["lenses"])[0]["n_src_active"] > 3000  # of 3600
+        build.append(qlx_ctx.kernel_time("lbkernel")[0])
+        ahead.append(qlx_ctx.kernel_time("lbuild")[0] - build[-1])
+    assert min(ahead) < min(build), (min(ahead), min(build))
