@@ -2935,7 +2935,7 @@ __device__ void tri_bwd(const T* L, int ld, int nb, const T* W, T* sx, T (*part)
 // 3712 mixed 6.6 -> 7.9 ms, 100 FP64 1.34 -> 1.42, so these keep the one workgroup.  The vector stands in slot 6 of the item's vectors, in the factor's type.
 #define PAN 256
 #define SOLVE_ONE_B 96      // items from which one workgroup each is the better form,
-#define SOLVE_ONE_LD 8192   // for factors whose vector fits LDS beside the partial sums (107 KB of FP64)
+// for factors up to QLX_SOLVE_ONE_LD, whose vector fits LDS beside the partial sums (107 KB of FP64)
 #define SOLVE_ONE_LDS(ld) (16 * PAN + 16 * (TS + 1) + TS + (size_t)(ld))
 template <typename T>
 __device__ __forceinline__ T* solve_vec(const BatchDev& bd, const ItemMeta& M) { return (T*)(bd.vec + M.vec_off + 6 * (size_t)M.ldN); }
@@ -3129,7 +3129,7 @@ template <typename T>
 static void launch_solve(hipStream_t s, const BatchDev& bd, int max_ld, int mode, bool one)
 {
     const int np = (max_ld + PAN - 1) / PAN;
-    if (one && max_ld <= SOLVE_ONE_LD) {
+    if (one && max_ld <= QLX_SOLVE_ONE_LD) {
         allow_big_lds((const void*)k_solve_one_b<T>);
         hipLaunchKernelGGL(k_solve_one_b<T>, dim3(1, bd.B), dim3(1024), SOLVE_ONE_LDS(max_ld) * sizeof(T), s, bd, mode);
         return;
@@ -3355,16 +3355,19 @@ __global__ void __launch_bounds__(1024) k_refine_check_b(BatchDev bd, int final_
     for (int c = tid; c < ld; c += 1024) v[c] = (c < n) ? (float)r[c] : 0.0f;
 }
 
-void launch_refine_b(hipStream_t s, const BatchDev& bd, int max_ld, int iters, double tol)
+void launch_refine_check_b(hipStream_t s, const BatchDev& bd, int max_ld, int final_check, double tol)
 {
     const int nb = max_ld / TS;
-    for (int it = 0; it <= iters; it++) {
-        hipLaunchKernelGGL(k_resid_rows_b, dim3(nb, bd.B), dim3(256), 0, s, bd);
-        hipLaunchKernelGGL(k_resid_cols_b, dim3(nb, bd.B), dim3(64), 0, s, bd);
-        hipLaunchKernelGGL(k_refine_check_b, dim3(1, bd.B), dim3(1024), 0, s, bd, it == iters ? 1 : 0, tol);
-        // steps after the first are for the few items still above the tolerance: one launch each
-        if (it < iters) launch_solve<float>(s, bd, max_ld, 1, it > 0 || bd.B >= SOLVE_ONE_B);
-    }
+    hipLaunchKernelGGL(k_resid_rows_b, dim3(nb, bd.B), dim3(256), 0, s, bd);
+    hipLaunchKernelGGL(k_resid_cols_b, dim3(nb, bd.B), dim3(64), 0, s, bd);
+    hipLaunchKernelGGL(k_refine_check_b, dim3(1, bd.B), dim3(1024), 0, s, bd, final_check, tol);
+}
+
+void launch_refine_step_b(hipStream_t s, const BatchDev& bd, int max_ld, int step)
+{
+    // steps after the first are for the few items still above the tolerance: one workgroup each, in one
+    // launch, up to QLX_SOLVE_ONE_LD
+    launch_solve<float>(s, bd, max_ld, 1, step > 0 || bd.B >= SOLVE_ONE_B);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -268,7 +268,10 @@ void cholesky_batched(hipStream_t s, const MatDesc* d_mats, int n32, int n64, in
                       int panel_blocks = 0);
 void launch_logdets_b(hipStream_t s, const BatchDev& bd, int f32);
 void launch_trisolve_b(hipStream_t s, const BatchDev& bd, int max_ld, int f32);
-void launch_refine_b(hipStream_t s, const BatchDev& bd, int max_ld, int iters, double tol);
+// iterative refinement: the residual and each item's convergence test; one correction of the items that go on
+#define QLX_SOLVE_ONE_LD 8192  // systems up to here are corrected in one launch, larger ones panel by panel
+void launch_refine_check_b(hipStream_t s, const BatchDev& bd, int max_ld, int final_check, double tol);
+void launch_refine_step_b(hipStream_t s, const BatchDev& bd, int max_ld, int step);
 void launch_evidence_b(hipStream_t s, const BatchDev& bd, int max_img, int max_src);
 // copy each valid item's source amplitudes (reference order), model image and cell map into its
 // block of `keep` at meta.keep_off: [cells doubles] [s_pix doubles] [cells ints]
