@@ -308,7 +308,7 @@ def main():
         roof_syrk = {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_F16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_F16_TFLOPS, 4), "traffic": read_traffic("syrk_f16_c2_traffic"),
                      "kernel": "k_syrk_f16_b (F = Lb^T C Lb: FP16 pool, FP32 accumulation, 128x128 tiles over "
-                               "the strips a chunk's rows reach)",
+                               "the strips a chunk's rows reach; executed flops, four column strips at a time)",
                      "items_per_launch": st["n_items"], "flops_block_sparse_per_launch": st["syrk_exec_flops"],
                      "pool_bytes_per_launch": st["lb_bytes"], "avg_launch_ms": round(syrk_s * 1e3, 3)}
 

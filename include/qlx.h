@@ -342,8 +342,9 @@ int qlx_kernel_time(void *ctx, const char *name, double *ms, int *launches);
 /* Work counters of the last wave of the last qlx_eval (no reference counterpart; benchmark
  * accounting).  Sums over the wave's items unless noted:
  *   syrk_dense_flops   2*64*16^2 per (lower pair of 16-column strips, 64-row chunk) of a dense SYRK
- *   syrk_exec_flops    MFMA flops executed: the same per pair of 64 x 16 pool strips of one 64-row
- *                      chunk (one product each)
+ *   syrk_exec_flops    MFMA flops executed: the same per pair of strips multiplied, in FP64 the pairs of
+ *                      pool strips of one 64-row chunk, in MIXED four column strips at a time if one of
+ *                      them is held (the absent ones as zeros)
  *   syrk_alg_flops     N_img*N_src*(N_src+1) + 2*N_img*N_src (the F and D arithmetic)
  *   lb_bytes           bytes of the blurred lensing matrix strips written
  *   integrand_evals    NFW integrand evaluations of the ray shooting

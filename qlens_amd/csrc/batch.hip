@@ -665,7 +665,8 @@ __global__ void __launch_bounds__(256) k_chunk_cols_b(BatchDev bd)
     }
 }
 
-// the chunks' first slots in the item's pool (in strips), the item's strips and its strip pairs
+// the chunks' first slots in the item's pool (in strips), the item's strips and the strip pairs that its SYRK
+// multiplies
 __global__ void __launch_bounds__(1024) k_block_scan_b(BatchDev bd)
 {
     __shared__ int sh[40];
@@ -680,9 +681,23 @@ __global__ void __launch_bounds__(1024) k_block_scan_b(BatchDev bd)
     for (int t0 = 0; t0 < M.nkt; t0 += 1024) {
         const int t = t0 + threadIdx.x;
         int v = 0;
-        if (t < M.nkt)
-            for (int w = 0; w < M.nsw; w++) v += __popc(nz[(size_t)t * M.nsw + w]);
-        pairs += (unsigned long long)v * (v + 1) / 2;
+        if (M.cbs == 6) {  // FP64: the SYRK multiplies the pairs held
+            if (t < M.nkt)
+                for (int w = 0; w < M.nsw; w++) v += __popc(nz[(size_t)t * M.nsw + w]);
+            pairs += (unsigned long long)v * (v + 1) / 2;
+        } else if (t < M.nkt) {
+            // FP16: a wave takes four column strips together, absent ones as zeros: per four of which one is
+            // held, the strips held from their first on, times four
+            unsigned long long fours = 0, before = 0;
+            for (int w = 0; w < M.nsw; w++)
+                for (unsigned x = nz[(size_t)t * M.nsw + w], q = 0; q < 8; q++, x >>= 4)
+                    if (x & 15u) {
+                        fours++;
+                        before += v;
+                        v += __popc(x & 15u);
+                    }
+            pairs += 4 * (fours * v - before);
+        }
         const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
         int incl = wave_incl_scan(v);
         if (lane == 63) sh[wv] = incl;

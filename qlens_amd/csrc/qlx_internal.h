@@ -128,7 +128,7 @@ struct BatchDev {
     int* bfill;                 // s_cell+2: scatter cursors
     int* perm;                  // s_pix: active row at each row-order position
     unsigned long long* nevals; // 1 per item
-    unsigned long long* npairs; // 1 per item: pairs of strips of one chunk
+    unsigned long long* npairs; // 1 per item: strip pairs of one chunk that its SYRK multiplies
     long long s_pix, s_cell;
     // pools and outputs
     const ItemMeta* meta;

@@ -82,3 +82,23 @@ def test_chunk_support_costs_less_than_the_pool(qlx_ctx, thin, psf, precision):
         build.append(qlx_ctx.kernel_time("lbkernel")[0])
         ahead.append(qlx_ctx.kernel_time("lbuild")[0] - build[-1])
     assert min(ahead) < min(build), (min(ahead), min(build))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("src_n", [(5, 3), (9, 9), (20, 14)])
+def test_executed_flops_are_those_of_the_products(qlx_ctx, src_n):
+    """A PSF wider than the image: every chunk holds every strip (the last one with the data column), so the
+    products are known: FP64 multiplies the lower pairs, the mixed kernel each strip against four column
+    strips from the strip's own block of 64 columns down."""
+    case = _case(40, 44, 2, src_n, (89, 89), None)
+    case["srcgrid"] = (-0.7, 0.7, -0.7, 0.7)
+    n = src_n[0] * src_n[1]
+    strips = n // 16 + 1
+    pairs = {qlx.QLX_PREC_FP64: strips * (strips + 1) // 2,
+             qlx.QLX_PREC_MIXED: 4 * sum(strips - h for h in range(0, strips, 4))}
+    for precision, want in pairs.items():
+        qlx_ctx.load_workload(case, np.ones((40, 44)), precision=precision)
+        r = qlx_ctx.invert_image_surface_brightness_map(case["lenses"])[0]
+        st = qlx.get_stats(qlx_ctx)
+        assert r["n_src_active"] == n
+        assert st["syrk_exec_flops"] == want * st["rows_pad"] // 64 * 2 * 64 * 16 * 16
