@@ -1,6 +1,6 @@
 """FP64 factorizations at the sizes where their tiles, panels and bands end: F's blocked Cholesky
 (64-blocks padded to 128, 256-wide parts, narrow or wide panels) and R's banded one (bands from one to
-several blocks), against the oracle; and the same bits alone and in a batch large enough for the wide
+17 blocks, the widest a grid can have), against the oracle; and the same bits alone and in a batch large enough for the wide
 schedule."""
 import numpy as np
 import pytest
@@ -21,7 +21,7 @@ def _case(src_n):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("src_n", [(2, 2), (9, 7), (8, 8), (11, 11), (13, 10), (16, 16), (18, 14), (23, 22), (33, 31), (64, 6), (96, 8), (6, 64)])
+@pytest.mark.parametrize("src_n", [(2, 2), (9, 7), (8, 8), (11, 11), (13, 10), (16, 16), (18, 14), (23, 22), (33, 31), (64, 6), (96, 8), (6, 64), (130, 4), (512, 2)])
 def test_factor_sizes_match_oracle(qlx_ctx, src_n):
     case = _case(src_n)
     data = O.mock_image(case)

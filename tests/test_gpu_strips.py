@@ -1,7 +1,8 @@
 """The blurred-L pool's strips and the SYRK over them, at the sizes where strips, column blocks, chunks
 and the tap table end: chunks that span two ends of an image row (thin masks and images), PSFs of one pixel
-to wider than the padded tap table takes, source grids whose last strip, block and data column fall at
-every place, and more chunks than one list holds; against the oracle, FP64 and mixed."""
+to wider than the padded tap table takes, partly reached source grids of various sizes, and more chunks than
+one list holds (test_strips_match_oracle); whole source grids whose data column opens a strip or a column
+block of its own or closes one (test_data_column_at_every_edge); against the oracle, FP64 and mixed."""
 import numpy as np
 import pytest
 
@@ -11,6 +12,8 @@ from qlens_amd import workloads as W
 
 TOL = 1e-9         # FP64: the oracle's sums in another order
 TOL_MIXED = 0.1    # |delta ln E| of the mixed path's contract
+TOL_SRC = 2e-3     # mixed path's source: both factors of F and D hold entries rounded to 11 bits (2^-11 each),
+                   # and twice that for a regularized solve, which damps more than it amplifies
 
 
 def _psf(n, m):
@@ -64,6 +67,30 @@ def test_strips_match_oracle(qlx_ctx, args, precision):
         assert abs(r[k] - ref[k]) <= TOL * max(1.0, abs(ref[k])), k
     src = qlx_ctx.get_source()["src"]
     assert np.linalg.norm(src - arr["src"]) <= TOL * np.linalg.norm(arr["src"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("src_n,thin", [((4, 4), False), ((8, 8), False), ((16, 8), False), ((17, 15), False), ((16, 16), False),
+                                        ((24, 16), False), ((20, 20), True)])
+@pytest.mark.parametrize("precision", [qlx.QLX_PREC_FP64, qlx.QLX_PREC_MIXED])
+def test_data_column_at_every_edge(qlx_ctx, src_n, thin, precision):
+    """n_src a multiple of 16, 64, 128 and 256 and one less: a strip, a column block and a padded system that
+    hold the data column alone, or that it fills; up to four column blocks of the mixed path."""
+    case = W.c1()
+    case["src_n"] = src_n
+    case["mask"] = _thin(100, 100) if thin else None
+    data = O.mock_image(case)
+    ref, arr = O.invert(case, data)
+    qlx_ctx.load_workload(case, data, precision=precision)
+    r = qlx_ctx.invert_image_surface_brightness_map(case["lenses"])[0]
+    assert r["status"] == 0 and r["n_src_active"] == ref["n_src"] == src_n[0] * src_n[1]
+    err = np.linalg.norm(qlx_ctx.get_source()["src"] - arr["src"]) / np.linalg.norm(arr["src"])
+    if precision == qlx.QLX_PREC_MIXED:
+        assert abs(r["minus2lnE"] - ref["minus2lnE"]) / 2 < TOL_MIXED and err <= TOL_SRC
+        return
+    for k in ("minus2lnE", "chisq0", "logdetF", "logdetR"):
+        assert abs(r[k] - ref[k]) <= TOL * max(1.0, abs(ref[k])), k
+    assert err <= TOL
 
 
 @pytest.mark.gpu
