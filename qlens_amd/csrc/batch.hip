@@ -40,7 +40,6 @@ __device__ __forceinline__ void store_nt(uint4* p, const uint4& v)
     __builtin_nontemporal_store((u32x4_t){v.x, v.y, v.z, v.w}, (u32x4_t*)p);
 }
 #define TS 64
-#define LDSP 66
 
 // raise the dynamic-LDS limit of a kernel once per process (kernels are told apart by address)
 static void allow_big_lds(const void* kernel)
@@ -1278,7 +1277,8 @@ void launch_syrk_f64_b(hipStream_t s, const BatchDev& bd, int max_ncb)
 // workgroup per 128 x 128 lower tile of F.  A operand lane l holds A[i = l%16][8 consecutive k], B the
 // same with j; accumulator register v of lane l holds D[4*(l/16) + v][l%16].  Only the strips a chunk
 // holds are read (33 of 16 columns a chunk on the 200 x 200 / 60 x 60 workload against 8.5 blocks of
-// 128) and multiplied.  As in the FP64 kernel the operands come straight from the pool into registers,
+// 128); each row strip held is multiplied by all four of the wave's column strips if one of them is held,
+// the absent ones as zeros (1.5 times the products of the pairs held).  As in the FP64 kernel the operands come straight from the pool into registers,
 // SYRK_D chunks ahead, with no staging and no barrier: wave (kh, jh) takes rows 32 kh .. of every chunk for
 // the tile's columns 64 jh .. (16-byte loads: a wave's load occupies the L1 for 16 cycles whatever its
 // width, and four waves of 16 rows with 8-byte ones took 14.4 ms).  The two row halves' sums are added
@@ -1577,7 +1577,7 @@ __global__ void __launch_bounds__(256) k_copy_f_b(BatchDev bd)
 // thread takes a cell's five pairs that lie ahead of it: a pass over those entries instead of one over F
 // that gathered an R entry for each of its own (FP16 SYRK's store 17.7 -> 13.8 ms of the kernel per 256
 // items of 3600 cells, the FP64 pass 2.45 ms per 100).  R is held in the reference order, F in the
-// internal one.  FP32: the diagonal 64-tiles' upper halves too, and the diagonal in FP64 into Fdiag.
+// internal one.  FP32: the diagonal 64-tiles' upper halves too, and the diagonal, as rounded to FP32, into Fdiag.
 template <typename T>
 __global__ void __launch_bounds__(256) k_add_reg_b(BatchDev bd)
 {
@@ -1949,12 +1949,6 @@ __device__ __forceinline__ void split64_store(const f32x4_t (&r)[4], __bf16* H, 
         *(bf16x4_t*)&H[i * LPB + k] = xh;
         *(bf16x4_t*)&L[i * LPB + k] = __builtin_convertvector(r[h] - __builtin_convertvector(xh, f32x4_t), bf16x4_t);
     }
-}
-__device__ __forceinline__ void stage64_split(const float* P, int sp, __bf16* H, __bf16* L)
-{
-    f32x4_t r[4];
-    load64_regs(P, sp, r);
-    split64_store(r, H, L);
 }
 
 // an accumulator tile (mma64's layout: wave (wr, wc) holds quadrant rows wr*32.., columns wc*32..)
@@ -2684,9 +2678,11 @@ __global__ void __launch_bounds__(256) k_chol_trail_f64(const MatDesc* mats, int
 // 30.1; FP32 MFMA in the panel kernel then).  FP64: 1024-wide panels where there are many matrices (100
 // of 3712: 36.7 ms with 1024, 37.8 with 512, 40.1 with 256, which reads and writes the trailing matrix four
 // times as often), 256-wide ones for few (one of 3712: 2.15, 2.21 and 2.31 ms with 256, 512 and 1024: the
-// strips are launches on the serial chain); 60.9 and 4.3 ms with right-looking panels.  The schedule's
-// arithmetic does not depend on the panel's width or on the batch, so an item's factor is the same bits
-// alone and in any.
+// strips are launches on the serial chain).  The line counts the trailing tiles, so that one large matrix is on
+// the wide side; 256 against 1024: one of 8192 7.55 / 7.53 ms, one of 10 112 11.34 / 11.29, four of these 29.8 /
+// 28.4, eight of 3712 4.38 / 4.35, 32 of them 12.3 / 11.7.  (Right-looking panels: 100 of 3712 60.9 ms, one
+// 4.3.)  The schedule's arithmetic does not depend on the panel's width or on the batch, so an item's
+// factor is the same bits alone and in any.
 #define CHOL_WIDE 16384  // matrices x blocks^2 from which FP64 panels are wide
 #define QLX_CHOL_SUB 4  // 256-wide left-looking parts per panel by default
 template <typename T>
@@ -2802,7 +2798,7 @@ __device__ __forceinline__ T sum16(T v)
 
 // forward: x_kb = W_kb (b_kb - L[kb, 0:kb] x_{0:kb}); wave w owns rows w, w+16, w+32, w+48 of the block
 template <typename T>
-__device__ void tri_fwd(const T* L, int ld, int nb, const T* W, T* sx, T (*part)[TS + 1], T* rhs)
+__device__ void tri_fwd(const T* L, int ld, int nb, const T* W, T* sx, T* rhs)
 {
     constexpr int VW = 16 / sizeof(T);
     typedef T P __attribute__((ext_vector_type(VW)));
@@ -2947,7 +2943,11 @@ __device__ void tri_bwd(const T* L, int ld, int nb, const T* W, T* sx, T (*part)
 // A solve reads its factor once; one workgroup gets the 55-110 GB/s of its CU, a launch per panel costs a
 // chain of a triangle and a product (~20 us) each.  The stage, one workgroup -> launches: 6 items of 10 000
 // mixed 12.2 -> 3.2 ms, one of 3712 mixed 1.21 -> 0.65, FP64 0.62 -> 0.31; one -> launches: 256 items of
-// 3712 mixed 6.6 -> 7.9 ms, 100 FP64 1.34 -> 1.42, so these keep the one workgroup.  The vector stands in slot 6 of the item's vectors, in the factor's type.
+// 3712 mixed 6.6 -> 7.9 ms, 100 FP64 1.34 -> 1.42, so these keep the one workgroup.  The line, by panels
+// against one workgroup each: of 3712, 64 items mixed 2.38 against 2.84 ms, 96 3.28 / 3.45, 128 4.00 / 3.70
+// (FP64 0.92 / 1.25, 1.29 / 1.35, 1.56 / 1.47); of 1024 the one workgroup is the better form at every
+// count, by at most 0.05 ms (8 items mixed 0.232 / 0.222, 96 0.552 / 0.508), so the size does not enter.
+// The vector stands in slot 6 of the item's vectors, in the factor's type.
 #define PAN 256
 #define SOLVE_ONE_B 96      // items from which one workgroup each is the better form,
 // for factors up to QLX_SOLVE_ONE_LD, whose vector fits LDS beside the partial sums (107 KB of FP64)
@@ -3068,7 +3068,6 @@ __global__ void __launch_bounds__(1024) k_solve_bwd_b(BatchDev bd, int s, int mo
 __global__ void __launch_bounds__(1024) k_solve_fwd_b(BatchDev bd, int s)
 {
     __shared__ __align__(16) float sx[PAN];
-    __shared__ float tpart[16][TS + 1];
     __shared__ float rhs[TS];
     const int item = blockIdx.y;
     const ItemMeta& M = bd.meta[item];
@@ -3088,7 +3087,7 @@ __global__ void __launch_bounds__(1024) k_solve_fwd_b(BatchDev bd, int s)
         sx[c] = v[q0 + c];
     }
     __syncthreads();
-    if (blockIdx.x == 0) tri_fwd<float>(L + (size_t)q0 * ld + q0, ld, nq / TS, (const float*)(bd.winv + M.w_off) + (size_t)q0 * TS, sx, tpart, rhs);
+    if (blockIdx.x == 0) tri_fwd<float>(L + (size_t)q0 * ld + q0, ld, nq / TS, (const float*)(bd.winv + M.w_off) + (size_t)q0 * TS, sx, rhs);
     if (c < nq) v[q0 + c] = sx[c];
 }
 
@@ -3114,7 +3113,7 @@ __global__ void __launch_bounds__(1024) k_solve_one_b(BatchDev bd, int mode)
         if (mode)
             for (int P = 0; P < np; P++) {
                 const int p0 = P * PAN;
-                tri_fwd<T>(L + (size_t)p0 * ld + p0, ld, min(PAN, ld - p0) / TS, W + (size_t)p0 * TS, sx + p0, tpart, rhs);
+                tri_fwd<T>(L + (size_t)p0 * ld + p0, ld, min(PAN, ld - p0) / TS, W + (size_t)p0 * TS, sx + p0, rhs);
                 const int r = (tid >> 6) + 16 * ((tid & 63) >> 2);
                 for (int q0 = p0 + PAN; q0 < ld; q0 += PAN) {
                     const int nq = min(PAN, ld - q0);

@@ -10,7 +10,8 @@ from qlens_amd import qlx
 from qlens_amd import workloads as W
 
 TOL = 1e-9          # FP64: the oracle's sums in another order
-TOL_MIXED = 1e-4    # mixed: refined to an FP64 residual of 1e-10 of the right side, on systems of condition below 1e6
+TOL_MIXED = 1e-4    # mixed: refined to an FP64 residual of 1e-10 of the right side, on systems of condition below 1e6,
+                    # formed from entries rounded to 11 bits (2^-11, averaged over the rows that a cell is seen in)
 
 
 @pytest.mark.gpu
