@@ -770,8 +770,9 @@ void launch_row_support_b(hipStream_t s, const BatchDev& bd, int max_nkt, int ma
 //               an MFMA operand; entries x = Lb sqrt(c_r) s16 rounded once (s16 a power of two, |x| <=
 //               2^14).
 // Column n_src carries the data: d (FP64) or d sqrt(c_r) s16 (FP16).  256 items of the 200 x 200 / 60 x 60
-// workload: 9.8 ms with half blocks of 64 columns shared by the four waves and stored whole (12.8 GB),
-// 6.7 on strips (5.6 GB), both FP16; bound by its LDS traffic (a broadcast and 64 tap reads per kept entry).
+// workload, FP16: 10.0 ms with half blocks of 64 columns shared by the four waves and stored whole (13.0 GB) and
+// the columns found in this kernel; 6.9 on strips (6.0 GB) after 1.1 in k_chunk_cols_b.  Bound by its LDS
+// traffic (a broadcast and 64 tap reads per kept entry).
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ uint16_t f32_to_f16_rne(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
 
@@ -2942,7 +2943,7 @@ __device__ void tri_bwd(const T* L, int ld, int nb, const T* W, T* sx, T (*part)
 //     themselves and the launches' tails would only idle it.
 // A solve reads its factor once; one workgroup gets the 55-110 GB/s of its CU, a launch per panel costs a
 // chain of a triangle and a product (~20 us) each.  The stage, one workgroup -> launches: 6 items of 10 000
-// mixed 12.2 -> 3.2 ms, one of 3712 mixed 1.21 -> 0.65, FP64 0.62 -> 0.31; one -> launches: 256 items of
+// mixed 12.2 -> 3.0 ms, one of 3712 mixed 1.21 -> 0.65, FP64 0.62 -> 0.31; one -> launches: 256 items of
 // 3712 mixed 6.6 -> 7.9 ms, 100 FP64 1.34 -> 1.42, so these keep the one workgroup.  The line, by panels
 // against one workgroup each: of 3712, 64 items mixed 2.38 against 2.84 ms, 96 3.28 / 3.45, 128 4.00 / 3.70
 // (FP64 0.92 / 1.25, 1.29 / 1.35, 1.56 / 1.47); of 1024 the one workgroup is the better form at every
